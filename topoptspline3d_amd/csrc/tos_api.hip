@@ -1818,7 +1818,8 @@ void coarse_alloc(Ctx& c) {
   c.cmap = dalloc<int>(c, cmap.size());
   upload(c.stream, c.cmap, cmap.data(), cmap.size() * sizeof(int));
   c.cinv = dalloc<double>(c, (size_t)c.cn * c.cn);
-  c.cwork = dalloc<double>(c, (size_t)c.cn * kGJB * 2 + kGJB * kGJB + c.cn);
+  // scratch of the factorisation: the sweep's second matrix, two pivot tiles, the diagonal
+  c.cwork = dalloc<double>(c, (size_t)c.cn * c.cn + 2 * kGJB * kGJB + c.cn);
   c.cflag = dalloc<int>(c, 1);
   if (c.floating && c.cn) {
     // the rigid motions of the coarsest nodes (coordinates relative to their centroid; a
@@ -1869,7 +1870,14 @@ int coarse_factor(Ctx& c, bool from32) {
   Level& L = c.L.back();
   const int n = c.cn, nnode = n / 3;
   if (from32 && !c.cinv32) c.cinv32 = dalloc<double>(c, (size_t)n * n);
-  double* A = from32 ? c.cinv32 : c.cinv;
+  // the sweep's steps alternate between the result and the second matrix: start where the
+  // last step ends in the result
+  double* const out = from32 ? c.cinv32 : c.cinv;
+  const int steps = (n + kGJB - 1) / kGJB;
+  double* A = (steps & 1) ? c.cwork : out;
+  double* B = (steps & 1) ? out : c.cwork;
+  double* Dinv[2] = {c.cwork + (size_t)n * n, c.cwork + (size_t)n * n + kGJB * kGJB};
+  double* diag0 = Dinv[1] + kGJB * kGJB;
   hipLaunchKernelGGL(k_zero<double>, dim3(nblk((int64_t)n * n)), dim3(256), 0, c.stream, A, (int64_t)n * n);
   if (from32)
     hipLaunchKernelGGL(k_coarse_assemble<float>, dim3(nblk((int64_t)nnode * 27)), dim3(256), 0, c.stream, L.v,
@@ -1879,10 +1887,6 @@ int coarse_factor(Ctx& c, bool from32) {
     hipLaunchKernelGGL(k_coarse_assemble<double>, dim3(nblk((int64_t)nnode * 27)), dim3(256), 0, c.stream, L.v,
                        (const int64_t*)c.cidx, nnode, (const int*)c.cmap, (const int*)L.slot,
                        (const double*)L.st64, L.NS, A, n);
-  double* Dinv = c.cwork;
-  double* Cp = Dinv + kGJB * kGJB;
-  double* R = Cp + (size_t)n * kGJB;
-  double* diag0 = R + (size_t)n * kGJB;
   hipLaunchKernelGGL(k_symmetrize, dim3(nblk((int64_t)n * n)), dim3(256), 0, c.stream, A, n, diag0);
   if (c.floating && c.crig_m) {
     // null space of a floating body: factor A + alpha R R^T (alpha = mean diagonal); for a
@@ -1896,14 +1900,12 @@ int coarse_factor(Ctx& c, bool from32) {
                        (const double*)c.crig, c.crig_m, alpha);
   }
   HIPCHK(hipMemsetAsync(c.cflag, 0, sizeof(int), c.stream));
-  for (int K0 = 0; K0 < n; K0 += kGJB) {
-    const int b = std::min(kGJB, n - K0);
-    hipLaunchKernelGGL(k_gj_pivot, dim3(1), dim3(64), 0, c.stream, A, n, K0, b, Dinv, (const double*)diag0,
-                       c.cflag);
-    hipLaunchKernelGGL(k_gj_panel, dim3(nblk((int64_t)n * b)), dim3(256), 0, c.stream, (const double*)A, n, K0,
-                       b, (const double*)Dinv, Cp, R);
-    hipLaunchKernelGGL(k_gj_update, dim3(nblk((int64_t)n * n)), dim3(256), 0, c.stream, A, n, K0, b,
-                       (const double*)Dinv, (const double*)Cp, (const double*)R);
+  hipLaunchKernelGGL(k_gj_first, dim3(1), dim3(256), 0, c.stream, (const double*)A, n, Dinv[0], (const double*)diag0,
+                     c.cflag);
+  for (int K = 0; K < steps; ++K) {
+    hipLaunchKernelGGL(k_gj_step, dim3(steps, steps), dim3(256), 0, c.stream, (const double*)A, B, n, K,
+                       (const double*)Dinv[K & 1], Dinv[(K + 1) & 1], (const double*)diag0, c.cflag);
+    std::swap(A, B);
   }
   LAUNCH_CHECK();
   int flag = 0;

@@ -198,7 +198,7 @@ struct Ctx {
   int64_t* cidx = nullptr;      // padded node index of each coarse unknown node
   double* cinv = nullptr;       // -A^{-1} after the sweep (cn x cn), from the FP64 stencils
   double* cinv32 = nullptr;     // the same from the FP32-built stencils (Galerkin precision 1)
-  double* cwork = nullptr;      // panel buffers
+  double* cwork = nullptr;      // factorisation scratch (see coarse_alloc)
   int* cflag = nullptr;         // singular pivot flag
   int* cmap = nullptr;          // padded coarsest node -> compact node index or -1
   void* stage = nullptr;        // host<->device conversion buffer
