@@ -1,0 +1,42 @@
+"""Grouping of the surface points by knot cell and its gradient sums, against the oracle, at
+the sizes where they can go wrong: cells of more points than a wavefront has lanes, spline
+orders whose k^3 block is smaller and larger than a wavefront, boxes without any point, and
+buffers reused after a larger and a smaller lattice.
+
+Both sides sum the same FP64 products, in another order; the results are FP32.  A gradient
+sums at most a few thousand terms of one sign pattern, so 1e-5 of the largest entry (100
+FP32 roundings) bounds the difference."""
+import numpy as np
+import pytest
+
+from test_gpu_surface import coeffs_for, hip, pair  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("mode,order,param,cells", [(1, 4, 8, (90, 24, 90)), (1, 2, 4, (40,)), (1, 5, 5, (60,)),
+                                                    (0, 3, 5, (70, 12)), (1, 3, 16, (64,))])
+def test_gradients_match_oracle(hip, mode, order, param, cells):  # noqa: F811
+    nx, ny, nz = 28, 20, 24
+    (o, g), n = pair(hip, nx, ny, nz, mode, order, param)
+    cf = coeffs_for(o, nx, ny, nz, mode, order, param)
+    for c in (o, g):
+        c.set_coeffs(cf)
+    for m in cells:
+        so, sg = (c.surface_constraints(cells=m, beta=8.0, ss_mode=4, drip_mode=7, drip_beta=4.0, drip_mu=2.0,
+                                        drip_beta_scale=1.0) for c in (o, g))
+        print(mode, order, param, m, sg, flush=True)
+        assert so["n_points"] == sg["n_points"]
+        for which in (2, 3):
+            go, gg = o.coeff_sens(which), g.coeff_sens(which)
+            assert np.abs(gg - go).max() <= 1e-5 * max(np.abs(go).max(), 1e-30), (m, which)
+
+
+def test_a_box_without_surface_points(hip):  # noqa: F811
+    (o, g), n = pair(hip, 12, 9, 10, 1, 4, 4)
+    cf = np.linspace(0.05, 0.3, n, dtype=np.float32)  # below the level everywhere
+    for c in (o, g):
+        c.set_coeffs(cf)
+        s = c.surface_constraints(cells=20, beta=8.0)
+        assert s["n_points"] == 0
+        assert not np.any(c.coeff_sens(2)) and not np.any(c.coeff_sens(3))

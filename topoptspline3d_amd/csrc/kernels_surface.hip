@@ -484,53 +484,62 @@ __global__ __launch_bounds__(256) void k_sf_fold(const double* __restrict__ part
   }
 }
 
-// per point and axis, the k coefficient indices and basis values / d / d2 (sf_axis), once:
-// bidx[(3 t + a) * 8 + q] (-1 past k or outside the spline's range),
-// bN[((3 t + a) * 3 + d) * 8 + q]
+// Per point and axis, once: the first coefficient index bidx[3 t + a] of its span (-1 outside
+// the spline's range) and the basis values / d / d2 of the k coefficients from it,
+// bN[((3 t + a) * 3 + d) * 8 + i] for coefficient bidx + i: the terms of sf_axis whose
+// (possibly clamped, hence repeated) index it is, summed in term order.
 __global__ void k_sf_basis(SfAxes S, int64_t n, const double* __restrict__ pts, int* __restrict__ bidx,
                            double* __restrict__ bN) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  for (int a = 0; a < 3; ++a) {
-    int idx[8];
-    double N[3][8];
-    const bool ok = sf_axis(S.a[a], pts[3 * t + a], idx, N);
-    for (int q = 0; q < 8; ++q) {
-      const bool use = ok && q < S.a[a].k;
-      bidx[(3 * t + a) * 8 + q] = use ? idx[q] : -1;
-      for (int d = 0; d < 3; ++d) bN[((3 * t + a) * 3 + d) * 8 + q] = use ? N[d][q] : 0.0;
+  const int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (u >= 3 * n) return;
+  const int a = (int)(u % 3);
+  int idx[8];
+  double N[3][8];
+  const SfAxis A = a == 0 ? S.a[0] : a == 1 ? S.a[1] : S.a[2];
+  const bool ok = sf_axis(A, pts[u], idx, N);
+  bidx[u] = ok ? idx[0] : -1;
+  for (int d = 0; d < 3; ++d)
+    for (int i = 0; i < 8; ++i) {
+      double s = 0;
+      if (ok)
+        for (int q = 0; q < A.k; ++q)
+          if (idx[q] - idx[0] == i) s += N[d][q];
+      bN[(u * 3 + d) * 8 + i] = s;
     }
-  }
-}
-
-// the contributions d/dc of coefficient index ci along axis a at point t (sf_basis_at from
-// the per-point table): sum over the terms q whose (possibly clamped) index equals ci
-__device__ __forceinline__ void sf_basis_tab(const int* __restrict__ bidx, const double* __restrict__ bN, int64_t t,
-                                             int a, int ci, double out[3]) {
-  out[0] = out[1] = out[2] = 0;
-  const int* ix = bidx + (3 * t + a) * 8;
-  const double* nn = bN + (3 * t + a) * 24;
-  for (int q = 0; q < 8; ++q)
-    if (ix[q] == ci)
-      for (int d = 0; d < 3; ++d) out[d] += nn[d * 8 + q];
 }
 
 // The coefficient gradients gather over points grouped by knot cell: a point's cell is the
 // first coefficient index of its span along each axis (clamped into the coefficient range,
 // sf_axis), and every coefficient the point touches lies in the k^3 block that starts at
-// that cell, so coefficient c gathers from the cells c - [0, k)^3.  key[t] = the cell
-// (-1 outside the spline's range), cnt[cell] += 1.
+// its cell.  cnt[cell] = points of the cell (order-independent integer counts).
 __global__ void k_sf_cell_count(int64_t n, int ncx, int ncy, const int* __restrict__ bidx, int* __restrict__ key,
                                 int* __restrict__ cnt) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n) return;
-  const int bx = bidx[(3 * t + 0) * 8], by = bidx[(3 * t + 1) * 8], bz = bidx[(3 * t + 2) * 8];
+  const int bx = bidx[3 * t], by = bidx[3 * t + 1], bz = bidx[3 * t + 2];
   int c = -1;
   if (bx >= 0 && by >= 0 && bz >= 0) {
     c = bx + ncx * (by + ncy * bz);
     atomicAdd(&cnt[c], 1);
   }
   key[t] = c;
+}
+
+// The cells that hold points get consecutive slots: slot[cell] (-1: empty), scell[slot].
+// Which slot a cell gets depends on scheduling; it only names a place in `part` below.
+__global__ void k_sf_cell_slots(int64_t ncell, const int* __restrict__ cnt, int* __restrict__ nslot,
+                                int* __restrict__ slot, int* __restrict__ scell) {
+  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const bool has = c < ncell && cnt[c] > 0;
+  const unsigned long long m = __ballot(has);
+  const int lane = threadIdx.x & 63;
+  int base = 0;
+  if (m && lane == __ffsll((unsigned long long)m) - 1) base = atomicAdd(nslot, __popcll(m));
+  if (m) base = __shfl(base, __ffsll((unsigned long long)m) - 1, 64);
+  if (c >= ncell) return;
+  const int s = base + __popcll(m & ((1ull << lane) - 1));
+  slot[c] = has ? s : -1;
+  if (has) scell[s] = (int)c;
 }
 
 // list[start[cell] ..) = the cell's points; cur (zeroed) hands out the slots in arrival
@@ -542,50 +551,48 @@ __global__ void k_sf_cell_fill(int64_t n, const int* __restrict__ key, const int
   list[start[key[t]] + atomicAdd(&cur[key[t]], 1)] = (int)t;
 }
 
-__global__ void k_sf_cell_sort(int64_t ncell, const int* __restrict__ start, int* __restrict__ list) {
-  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= ncell) return;
-  const int b = start[c], e = start[c + 1];
-  for (int i = b + 1; i < e; ++i) {  // insertion sort: a cell holds a few points
+// One wavefront per occupied cell: every lane ranks its points among the cell's (distinct)
+// points and stores them there.  A lattice finer than the knots puts hundreds of points in
+// a cell: one thread per cell sorting in place took 6.7 ms on 128 cells over 128 x 64 x 64
+// voxels, this 0.08 ms.
+__global__ __launch_bounds__(256) void k_sf_cell_sort(const int* __restrict__ nslot, const int* __restrict__ scell,
+                                                      const int* __restrict__ start, const int* __restrict__ list,
+                                                      int* __restrict__ sorted) {
+  const int s = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * 256 + threadIdx.x) >> 6));
+  if (s >= *nslot) return;  // whole wavefronts
+  const int c = scell[s], b = start[c], e = start[c + 1];
+  for (int i = b + (int)(threadIdx.x & 63); i < e; i += 64) {
     const int v = list[i];
-    int p = i - 1;
-    while (p >= b && list[p] > v) {
-      list[p + 1] = list[p];
-      --p;
-    }
-    list[p + 1] = v;
+    int r = b;
+    for (int j = b; j < e; ++j) r += list[j] < v ? 1 : 0;
+    sorted[r] = v;
   }
 }
 
-// gss/gdr[c] = factor * sum over the points of the cells c - [0, k)^3 of w . (basis
-// derivatives of c).  One wavefront per coefficient: lane l takes the window cells l,
-// l + 64, ... (cell order, then point order), and lane 0 sums the 64 lanes in a fixed
-// butterfly order, so the result does not depend on scheduling.
-__global__ __launch_bounds__(256) void k_sf_grad(SfAxes S, int64_t ncoef, const int* __restrict__ start,
-                                                 const int* __restrict__ list, const int* __restrict__ bidx,
-                                                 const double* __restrict__ bN, const double* __restrict__ wss,
-                                                 const double* __restrict__ wdr, double fss, double fdr,
-                                                 float* __restrict__ gss, float* __restrict__ gdr) {
-  const int64_t j = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const int lane = threadIdx.x & 63;
-  if (j >= ncoef) return;  // whole wavefronts
-  const int k = S.a[0].k, ncx = S.a[0].nc, ncy = S.a[1].nc;
-  const int ci[3] = {(int)(j % ncx), (int)((j / ncx) % ncy), (int)(j / ((int64_t)ncx * ncy))};
-  double a_ss = 0, a_dr = 0;
-  int seen = 0;
-  for (int w = lane; w < k * k * k; w += 64) {
-    const int bx = ci[0] - w % k, by = ci[1] - (w / k) % k, bz = ci[2] - w / (k * k);
-    if (bx < 0 || by < 0 || bz < 0) continue;
-    const int64_t cell = bx + (int64_t)ncx * (by + (int64_t)ncy * bz);
-    const int e = start[cell + 1];
-    for (int p = start[cell]; p < e; ++p) {
+// part[(slot k^3 + w) 2 ..) = the sums over a cell's points of w . (basis derivatives) for
+// the coefficient at offset w = i + k (j + k l) of the cell's block, self-support and drip.
+// One wavefront per occupied cell, lane = offset (all 64 busy at order 4), points in
+// ascending order; touch[c] marks the coefficients that any cell reaches.
+__global__ __launch_bounds__(256) void k_sf_cell_grad(SfAxes S, const int* __restrict__ nslot,
+                                                      const int* __restrict__ scell, const int* __restrict__ start,
+                                                      const int* __restrict__ list, const double* __restrict__ bN,
+                                                      const double* __restrict__ wss, const double* __restrict__ wdr,
+                                                      double* __restrict__ part, uint8_t* __restrict__ touch) {
+  const int s = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * 256 + threadIdx.x) >> 6));
+  if (s >= *nslot) return;  // whole wavefronts
+  const int k = S.a[0].k, ncx = S.a[0].nc, ncy = S.a[1].nc, ncz = S.a[2].nc, kk = k * k * k;
+  const int c = scell[s], b = start[c], e = start[c + 1];
+  const int cx = c % ncx, cy = (c / ncx) % ncy, cz = c / (ncx * ncy);
+  for (int w = threadIdx.x & 63; w < kk; w += 64) {
+    const int i = w % k, j = (w / k) % k, l = w / (k * k);
+    double a_ss = 0, a_dr = 0;
+    for (int p = b; p < e; ++p) {
       const int64_t t = list[p];
-      ++seen;
-      double X[3], Y[3], Z[3];
-      sf_basis_tab(bidx, bN, t, 0, ci[0], X);
+      const double* nn = bN + 72 * t;
+      const double X[3] = {nn[i], nn[8 + i], nn[16 + i]};
+      const double Y[3] = {nn[24 + j], nn[32 + j], nn[40 + j]};
+      const double Z[3] = {nn[48 + l], nn[56 + l], nn[64 + l]};
       if (X[0] == 0 && X[1] == 0 && X[2] == 0) continue;
-      sf_basis_tab(bidx, bN, t, 1, ci[1], Y);
-      sf_basis_tab(bidx, bN, t, 2, ci[2], Z);
       const double gx = X[1] * Y[0] * Z[0], gy = X[0] * Y[1] * Z[0], gz = X[0] * Y[0] * Z[1];
       const double* ws = &wss[3 * t];
       const double* wd = &wdr[6 * t];
@@ -593,16 +600,54 @@ __global__ __launch_bounds__(256) void k_sf_grad(SfAxes S, int64_t ncoef, const 
       a_dr += wd[0] * gx + wd[1] * gy + wd[2] * gz + wd[3] * X[2] * Y[0] * Z[0] + wd[4] * X[0] * Y[2] * Z[0] +
               wd[5] * X[1] * Y[1] * Z[0];
     }
+    part[2 * ((int64_t)s * kk + w)] = a_ss;
+    part[2 * ((int64_t)s * kk + w) + 1] = a_dr;
+    if (cx + i < ncx && cy + j < ncy && cz + l < ncz)
+      touch[(cx + i) + (int64_t)ncx * ((cy + j) + (int64_t)ncy * (cz + l))] = 1;
   }
-  if (__ballot(seen > 0) != 0) {
+}
+
+// gss/gdr[c] = factor * the sums of the cells c - [0, k)^3 for c: lane l takes the window
+// offsets l, l + 64, ... and lane 0 sums the 64 lanes in a fixed butterfly order, so the
+// result does not depend on scheduling.  One wavefront per kSfGradC coefficients; those no
+// cell reaches (most of a large lattice) are only written.  Forming the point sums here,
+// lane = cell, left the lanes at their cells' different point counts: 2.6 ms on 128 cells
+// over 128 x 64 x 64 voxels, the two kernels together 0.27 ms.
+constexpr int kSfGradC = 8;
+__global__ __launch_bounds__(256) void k_sf_grad(SfAxes S, int64_t ncoef, const int* __restrict__ slot,
+                                                 const double* __restrict__ part, const uint8_t* __restrict__ touch,
+                                                 double fss, double fdr, float* __restrict__ gss,
+                                                 float* __restrict__ gdr) {
+  const int64_t j0 = (((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6) * kSfGradC;
+  const int lane = threadIdx.x & 63;
+  if (j0 >= ncoef) return;  // whole wavefronts
+  const int k = S.a[0].k, ncx = S.a[0].nc, ncy = S.a[1].nc, kk = k * k * k;
+  const bool mine = lane < kSfGradC && j0 + lane < ncoef;
+  const bool hit = mine && touch[j0 + lane] != 0;
+  if (mine && !hit) {
+    gss[j0 + lane] = (float)(fss * 0.0);
+    gdr[j0 + lane] = (float)(fdr * 0.0);
+  }
+  for (unsigned long long m = __ballot(hit); m; m &= m - 1) {
+    const int64_t j = j0 + __ffsll(m) - 1;
+    const int ci[3] = {(int)(j % ncx), (int)((j / ncx) % ncy), (int)(j / ((int64_t)ncx * ncy))};
+    double a_ss = 0, a_dr = 0;
+    for (int w = lane; w < kk; w += 64) {
+      const int bx = ci[0] - w % k, by = ci[1] - (w / k) % k, bz = ci[2] - w / (k * k);
+      if (bx < 0 || by < 0 || bz < 0) continue;
+      const int s = slot[bx + (int64_t)ncx * (by + (int64_t)ncy * bz)];
+      if (s < 0) continue;
+      a_ss += part[2 * ((int64_t)s * kk + w)];
+      a_dr += part[2 * ((int64_t)s * kk + w) + 1];
+    }
     for (int o = 1; o < 64; o <<= 1) {
       a_ss += __shfl_xor(a_ss, o, 64);
       a_dr += __shfl_xor(a_dr, o, 64);
     }
-  }
-  if (lane == 0) {
-    gss[j] = (float)(fss * a_ss);
-    gdr[j] = (float)(fdr * a_dr);
+    if (lane == 0) {
+      gss[j] = (float)(fss * a_ss);
+      gdr[j] = (float)(fdr * a_dr);
+    }
   }
 }
 

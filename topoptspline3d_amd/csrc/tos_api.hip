@@ -4044,6 +4044,10 @@ TOS_EXPORT int tos_surface_constraints(tos_ctx* c, const tos_surface_opts* o, to
       const int64_t nsb = ((int64_t)ncoef + kSfScanBlock - 1) / kSfScanBlock;
       C.sf_cbsum = dalloc<int>(C, nsb);
       C.sf_cboff = dalloc<int>(C, nsb + 1);
+      C.sf_slot = dalloc<int>(C, ncoef);
+      C.sf_scell = dalloc<int>(C, ncoef);
+      C.sf_nslot = dalloc<int>(C, 1);
+      C.sf_touch = dalloc<uint8_t>(C, ncoef);
       C.sf_ncoef = (int64_t)ncoef;
     }
     {  // all coefficients equal: no surface; the driver's constants (utils/test_utils.cpp:1106-1113)
@@ -4139,16 +4143,23 @@ TOS_EXPORT int tos_surface_constraints(tos_ctx* c, const tos_surface_opts* o, to
     }
     if (C.sf_bcap < std::max<int64_t>(n, 1)) {
       C.sf_bcap = std::max<int64_t>(n, 1024) * 2;
-      C.sf_bidx = dalloc<int>(C, 24 * C.sf_bcap);
+      C.sf_bidx = dalloc<int>(C, 3 * C.sf_bcap);
       C.sf_bN = dalloc<double>(C, 72 * C.sf_bcap);
       C.sf_key = dalloc<int>(C, C.sf_bcap);
       C.sf_list = dalloc<int>(C, C.sf_bcap);
+      C.sf_sorted = dalloc<int>(C, C.sf_bcap);
     }
-    // points grouped by knot cell (count, scan, fill, per-cell sort), then the gather
-    const int64_t nc64 = (int64_t)ncoef;
+    // points grouped by knot cell (count, scan, fill, per-cell sort), the sums of every
+    // occupied cell (at most one cell per point), then the gather over the cells
+    const int64_t nc64 = (int64_t)ncoef, kk = (int64_t)C.sp_order * C.sp_order * C.sp_order;
+    const int64_t max_slots = std::min<int64_t>(n, nc64);
+    if (C.sf_pcap < 2 * kk * max_slots) {
+      C.sf_pcap = std::min<int64_t>(2 * max_slots, nc64) * 2 * kk;
+      C.sf_part = dalloc<double>(C, C.sf_pcap);
+    }
     hipLaunchKernelGGL(k_zero<int>, dim3(nblk(nc64)), dim3(256), 0, C.stream, C.sf_ccnt, nc64);
     if (n) {
-      hipLaunchKernelGGL(k_sf_basis, dim3(nblk(n)), dim3(256), 0, C.stream, S, n, (const double*)C.sf_pts,
+      hipLaunchKernelGGL(k_sf_basis, dim3(nblk(3 * n)), dim3(256), 0, C.stream, S, n, (const double*)C.sf_pts,
                          C.sf_bidx, C.sf_bN);
       hipLaunchKernelGGL(k_sf_cell_count, dim3(nblk(n)), dim3(256), 0, C.stream, n, C.nc[0], C.nc[1],
                          (const int*)C.sf_bidx, C.sf_key, C.sf_ccnt);
@@ -4162,15 +4173,24 @@ TOS_EXPORT int tos_surface_constraints(tos_ctx* c, const tos_surface_opts* o, to
       hipLaunchKernelGGL(k_sf_scan_apply, dim3(nsb), dim3(1024), 0, C.stream, (const int*)C.sf_ccnt, nc64,
                          (const int*)C.sf_cboff, C.sf_cstart);
     }
+    hipLaunchKernelGGL(k_zero<int>, dim3(1), dim3(256), 0, C.stream, C.sf_nslot, (int64_t)1);
+    hipLaunchKernelGGL(k_sf_cell_slots, dim3(nblk(nc64)), dim3(256), 0, C.stream, nc64, (const int*)C.sf_ccnt,
+                       C.sf_nslot, C.sf_slot, C.sf_scell);
     hipLaunchKernelGGL(k_zero<int>, dim3(nblk(nc64)), dim3(256), 0, C.stream, C.sf_ccnt, nc64);
-    if (n)
+    hipLaunchKernelGGL(k_zero<uint8_t>, dim3(nblk(nc64)), dim3(256), 0, C.stream, C.sf_touch, nc64);
+    if (n) {
       hipLaunchKernelGGL(k_sf_cell_fill, dim3(nblk(n)), dim3(256), 0, C.stream, n, (const int*)C.sf_key,
                          (const int*)C.sf_cstart, C.sf_ccnt, C.sf_list);
-    hipLaunchKernelGGL(k_sf_cell_sort, dim3(nblk(nc64)), dim3(256), 0, C.stream, nc64, (const int*)C.sf_cstart,
-                       C.sf_list);
-    hipLaunchKernelGGL(k_sf_grad, dim3(nblk(64 * nc64)), dim3(256), 0, C.stream, S, nc64, (const int*)C.sf_cstart,
-                       (const int*)C.sf_list, (const int*)C.sf_bidx, (const double*)C.sf_bN,
-                       (const double*)C.sf_wss, (const double*)C.sf_wdr, ss_fac, dr_fac, C.sscsens, C.dripcsens);
+      hipLaunchKernelGGL(k_sf_cell_sort, dim3(nblk(64 * max_slots)), dim3(256), 0, C.stream, (const int*)C.sf_nslot,
+                         (const int*)C.sf_scell, (const int*)C.sf_cstart, (const int*)C.sf_list, C.sf_sorted);
+      hipLaunchKernelGGL(k_sf_cell_grad, dim3(nblk(64 * max_slots)), dim3(256), 0, C.stream, S,
+                         (const int*)C.sf_nslot, (const int*)C.sf_scell, (const int*)C.sf_cstart,
+                         (const int*)C.sf_sorted, (const double*)C.sf_bN, (const double*)C.sf_wss,
+                         (const double*)C.sf_wdr, C.sf_part, C.sf_touch);
+    }
+    hipLaunchKernelGGL(k_sf_grad, dim3(nblk((nc64 + kSfGradC - 1) / kSfGradC * 64)), dim3(256), 0, C.stream, S, nc64,
+                       (const int*)C.sf_slot, (const double*)C.sf_part, (const uint8_t*)C.sf_touch, ss_fac, dr_fac,
+                       C.sscsens, C.dripcsens);
     LAUNCH_CHECK();
     HIPCHK(hipStreamSynchronize(C.stream));
     C.ss_value = ss_val;

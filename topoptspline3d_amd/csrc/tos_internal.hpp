@@ -249,10 +249,16 @@ struct Ctx {
   int* sf_tab_i = nullptr;   // per axis and lattice index: coefficient indices, basis values, flags
   double* sf_tab_v = nullptr;
   uint8_t* sf_tab_ok = nullptr;
-  int* sf_bidx = nullptr;    // per point and axis: coefficient indices and basis values (grown on demand)
+  int* sf_bidx = nullptr;    // per point and axis: first coefficient and basis values (grown on demand)
   double* sf_bN = nullptr;
   int* sf_key = nullptr;     // per point: knot cell (grown with sf_bidx)
-  int* sf_list = nullptr;    // points grouped by knot cell
+  int* sf_list = nullptr;    // points grouped by knot cell, in arrival and in point order
+  int* sf_sorted = nullptr;
+  int *sf_slot = nullptr, *sf_scell = nullptr;  // occupied cells: slot of a cell (-1 empty), cell of a slot
+  int* sf_nslot = nullptr;
+  uint8_t* sf_touch = nullptr;                  // coefficients reached by any point
+  double* sf_part = nullptr;                    // k^3 pairs of gradient sums per occupied cell
+  int64_t sf_pcap = 0;                          // doubles in sf_part
   int64_t sf_bcap = 0;
   int64_t sf_ncoef = 0;      // coefficient count the per-coefficient buffers below are sized for
   int *sf_ccnt = nullptr, *sf_cstart = nullptr;  // points per knot cell (then fill cursor), cell offsets
