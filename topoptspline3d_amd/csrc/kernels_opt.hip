@@ -449,29 +449,175 @@ __global__ __launch_bounds__(256) void k_oc_init_flat(const double* __restrict__
   }
 }
 
+// Where the OC density of one element lies, from a 32-bit estimate t of rho (gg/g)^damp that is
+// within 3e-5 of it (v_log_f32 and v_exp_f32 within an ulp over the admitted range
+// 1e-30 < gg/g < 1e30, damp <= 4): outside [lower, upper] by more than 1e-3 the clamp decides
+// the value, which is then the same float as oc_rho's; anything else (near the clamps, between
+// them, or not in range: NaN, infinities, tiny or non-positive densities) is kOcExact.
+enum { kOcLower = 0, kOcUpper = 1, kOcExact = 2 };
+__device__ __forceinline__ int oc_class(float r0, float s, double g, double inv_g, double move, float damp,
+                                        double rmin, float& val) {
+  const double gg = s > 0 ? 0.0 : -(double)s;
+  const float lo = (float)fmin(fmax((double)r0 - move, rmin), 1.0), hi = (float)fmin(fmax((double)r0 + move, rmin), 1.0);
+  const float x = (float)(gg * inv_g);
+  const bool zero = gg == 0.0 && g > 0.0, in = x > 1e-30f && x < 1e30f && damp <= 4.0f;
+  const float t = zero ? 0.0f : r0 * __builtin_amdgcn_exp2f(damp * __builtin_amdgcn_logf(x));
+  const bool ok = (zero || in) && r0 > 1e-30f && lo > 1e-30f;
+  const bool low = ok && t < lo * 0.999f, up = ok && t > hi * 1.001f;
+  val = low ? lo : hi;
+  return low ? kOcLower : (up ? kOcUpper : kOcExact);
+}
+
+// Calls body(valid, i, r0, s, shell) for the block's chunk of elements, four consecutive ones
+// per thread and step; body is called by whole waves (`valid` false past the end and for
+// inactive elements).  vec: 16-byte loads of rho and s, 4-byte loads of the masks.
+template <class F>
+__device__ __forceinline__ void oc_flat_chunk(int64_t n, int64_t chunk, bool vec, const uint8_t* act,
+                                              const uint8_t* shell, const float* rho, const float* s, F&& body) {
+  const int64_t i0 = (int64_t)blockIdx.x * chunk, i1 = min(n, i0 + chunk);
+  for (int64_t ib = i0; ib < i1; ib += 4 * 256) {
+    const int64_t i = ib + 4 * (int64_t)threadIdx.x;
+    float r[4] = {0, 0, 0, 0}, sv[4] = {0, 0, 0, 0};
+    uint32_t am = 0, sm = 0;
+    if (vec && i + 4 <= i1) {
+      const float4 a = *(const float4*)(rho + i), b = *(const float4*)(s + i);
+      am = act ? *(const uint32_t*)(act + i) : 0x01010101u;
+      sm = shell ? *(const uint32_t*)(shell + i) : 0u;
+      r[0] = a.x; r[1] = a.y; r[2] = a.z; r[3] = a.w;
+      sv[0] = b.x; sv[1] = b.y; sv[2] = b.z; sv[3] = b.w;
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (i + k < i1) {
+          r[k] = rho[i + k];
+          sv[k] = s[i + k];
+          am |= (uint32_t)(act ? act[i + k] : 1) << (8 * k);
+          sm |= (uint32_t)(shell ? shell[i + k] : 0) << (8 * k);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) body(((am >> (8 * k)) & 255u) != 0, i + k, r[k], sv[k], ((sm >> (8 * k)) & 255u) != 0);
+  }
+}
+
+// One trial of the flat OC: the block's sum of trial densities at g = scal[S_OC_G].
+// An FP64 pow per element bound the plain form (144 us a trial at 2^24 elements, 1.2 TB/s);
+// here oc_class settles the elements off the clamps and each wave collects the others in LDS
+// and evaluates them 64 at a time.  A block whose elements are all decided by clamps, the same
+// ones at both ends of the bracket (a threshold in between then gives the same density, the
+// update being monotone in the threshold), or all at the lower (upper) clamp at the lower
+// (upper) end, keeps its sum and reads no element: with a target that the move limit does not
+// reach nearly every block after the first trial.  A trial over all blocks now takes 37 us, one
+// over decided blocks 3; a call with a target out of reach 4.4 -> 0.34 ms.  state[b]: elements at the upper clamp at the
+// bracket's ends and in the last trial (-1: not known, or some not decided by a clamp), and the
+// number of elements that are neither inactive nor shell.
 __global__ __launch_bounds__(256) void k_oc_trial_flat(int64_t n, int64_t chunk, const uint8_t* __restrict__ act,
                                                        const uint8_t* __restrict__ shell, const float* __restrict__ rho,
                                                        const float* __restrict__ s, double move, double damp,
-                                                       double rmin, const double* __restrict__ scal,
-                                                       double* __restrict__ partial) {
+                                                       double rmin, double vgoal, int first, int vec,
+                                                       const double* __restrict__ scal, double* __restrict__ partial,
+                                                       short4* __restrict__ state) {
   if (scal[S_OC_DONE] != 0.0) return;
-  const double g = scal[S_OC_G];
-  const int64_t i0 = (int64_t)blockIdx.x * chunk, i1 = min(n, i0 + chunk);
+  __shared__ float2 queue[4][128];
+  const double g = scal[S_OC_G], inv_g = 1.0 / g;
+  short4 st = make_short4(-1, -1, -1, -1);  // lower end, upper end, last trial, free elements
+  if (!first) {
+    st = state[blockIdx.x];
+    const double V = scal[S_OC_V];
+    if (V > vgoal) st.x = st.z;
+    else if (V < vgoal) st.y = st.z;
+    if (st.x == 0 || (st.y >= 0 && (st.y == st.w || st.y == st.x))) {
+      st.z = st.x == 0 ? 0 : st.y;
+      __syncthreads();  // every thread has read the state
+      if (threadIdx.x == 0) state[blockIdx.x] = st;
+      return;
+    }
+  }
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  float2* q = queue[wv];
+  const float fdamp = (float)damp;
   double v = 0;
-  for (int64_t i = i0 + threadIdx.x; i < i1; i += 256)
-    if (!act || act[i]) v += (double)oc_rho(rho[i], s[i], g, move, damp, rmin, shell && shell[i]);
+  int nq = 0, up = 0, free_n = 0, exact = 0;
+  oc_flat_chunk(n, chunk, vec != 0, act, shell, rho, s, [&](bool valid, int64_t, float r0, float si, bool sh) {
+    float val = 1.0f;
+    int cls = kOcLower;
+    if (!sh) cls = oc_class(r0, si, g, inv_g, move, fdamp, rmin, val);
+    const bool ex = valid && !sh && cls == kOcExact;
+    if (valid && !ex) v += (double)val;
+    if (valid && !sh) {
+      ++free_n;
+      up += cls == kOcUpper;
+    }
+    const uint64_t m = __ballot(ex);
+    if (m) {
+      if (ex) q[nq + __popcll(m & ((1ull << lane) - 1))] = make_float2(r0, si);
+      nq += __popcll(m);
+      exact = 1;
+      if (nq >= 64) {
+        __threadfence_block();
+        nq -= 64;
+        const float2 e = q[nq + lane];
+        __threadfence_block();
+        v += (double)oc_rho(e.x, e.y, g, move, damp, rmin, false);
+      }
+    }
+  });
+  __threadfence_block();
+  if (lane < nq) v += (double)oc_rho(q[lane].x, q[lane].y, g, move, damp, rmin, false);
   v = block_sum256(v);
-  if (threadIdx.x == 0) partial[blockIdx.x] = v;
+  const double c = block_sum256((double)up + 65536.0 * free_n + 4294967296.0 * exact);
+  if (threadIdx.x == 0) {
+    partial[blockIdx.x] = v;
+    const int64_t k = (int64_t)c;
+    st.z = (k >> 32) ? -1 : (short)(k & 65535);
+    st.w = (short)((k >> 16) & 65535);
+    state[blockIdx.x] = st;
+  }
 }
 
 // active elements get the OC density of the final threshold, the others keep their input
-__global__ void k_oc_apply_flat(int64_t n, const uint8_t* __restrict__ act, const uint8_t* __restrict__ shell,
-                                const float* rho, const float* __restrict__ s, float* rho_out, double move,
-                                double damp, double rmin, const double* __restrict__ scal) {
-  const int64_t i = tid64();
-  if (i >= n) return;
-  const float r0 = rho[i];
-  rho_out[i] = (!act || act[i]) ? oc_rho(r0, s[i], scal[S_OC_G], move, damp, rmin, shell && shell[i]) : r0;
+// (rho_out may be rho: an element's input is read before its output is written, by one wave).
+// 119 -> 40 us at 2^24 elements, for the reason given at k_oc_trial_flat.
+__global__ __launch_bounds__(256) void k_oc_apply_flat(int64_t n, int64_t chunk, const uint8_t* __restrict__ act,
+                                                       const uint8_t* __restrict__ shell, const float* rho,
+                                                       const float* __restrict__ s, float* rho_out, double move,
+                                                       double damp, double rmin, int vec,
+                                                       const double* __restrict__ scal) {
+  __shared__ float2 queue[4][128];
+  __shared__ int qidx[4][128];
+  const double g = scal[S_OC_G], inv_g = 1.0 / g;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t i0 = (int64_t)blockIdx.x * chunk, i1 = min(n, i0 + chunk);
+  float2* q = queue[wv];
+  int* qi = qidx[wv];
+  const float fdamp = (float)damp;
+  int nq = 0;
+  oc_flat_chunk(n, chunk, vec != 0, act, shell, rho, s, [&](bool valid, int64_t i, float r0, float si, bool sh) {
+    float val = 1.0f;
+    int cls = kOcLower;
+    if (!sh) cls = oc_class(r0, si, g, inv_g, move, fdamp, rmin, val);
+    const bool ex = valid && !sh && cls == kOcExact;
+    if (i < i1 && !ex) rho_out[i] = valid ? val : r0;
+    const uint64_t m = __ballot(ex);
+    if (m) {
+      if (ex) {
+        const int k = nq + __popcll(m & ((1ull << lane) - 1));
+        q[k] = make_float2(r0, si);
+        qi[k] = (int)(i - i0);
+      }
+      nq += __popcll(m);
+      if (nq >= 64) {
+        __threadfence_block();
+        nq -= 64;
+        const float2 e = q[nq + lane];
+        const int k = qi[nq + lane];
+        __threadfence_block();
+        rho_out[i0 + k] = oc_rho(e.x, e.y, g, move, damp, rmin, false);
+      }
+    }
+  });
+  __threadfence_block();
+  if (lane < nq) rho_out[i0 + qi[lane]] = oc_rho(q[lane].x, q[lane].y, g, move, damp, rmin, false);
 }
 
 // ---------------------------------------------------------------------------------------

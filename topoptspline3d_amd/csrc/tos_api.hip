@@ -4796,7 +4796,8 @@ namespace {
 constexpr int kNoAllocChunk = 256 * 32;   // elements per block of the flat OC kernels
 constexpr int kNoAllocParts = 8192;       // block partials the scratch holds
 static_assert((int64_t)kNoAllocChunk * kNoAllocParts == TOS_NOALLOC_MAX_ELEMENTS, "capacity");
-// [0, 2*kNoAllocParts): partials (max |s| and active counts, then trial volumes);
+// [0, 2*kNoAllocParts): partials (max |s| and active counts, then trial volumes in the first
+// half and the blocks' clamp counts, 4 x 16 bits each, in the second);
 // [2*kNoAllocParts, +S_COUNT): the bisection scalars (S_OC_*, S_VOL = active count)
 static __device__ __align__(256) double scratch[2 * kNoAllocParts + S_COUNT];
 
@@ -4841,14 +4842,18 @@ TOS_EXPORT int tos_oc_update_noalloc(int64_t n, const uint8_t* active, const uin
   hipLaunchKernelGGL(k_absmax_count_flat, dim3(nb), dim3(256), 0, st, n, (int64_t)kNoAllocChunk, active, sens, nb,
                      part);
   hipLaunchKernelGGL(k_oc_init_flat, dim3(1), dim3(256), 0, st, (const double*)part, nb, scal);
+  // 16-byte loads where every array allows them; element by element otherwise
+  const int vec = ((uintptr_t)rho % 16 == 0 && (uintptr_t)sens % 16 == 0 && (uintptr_t)active % 4 == 0 &&
+                   (uintptr_t)shell % 4 == 0);
   for (int it = 0; it < 31; ++it) {
     hipLaunchKernelGGL(k_oc_trial_flat, dim3(nb), dim3(256), 0, st, n, (int64_t)kNoAllocChunk, active, shell, rho,
-                       sens, move, damp, rho_min, (const double*)scal, part);
+                       sens, move, damp, rho_min, vgoal, it == 0, vec, (const double*)scal, part,
+                       (short4*)(S + kNoAllocParts));
     hipLaunchKernelGGL(k_oc_decide, dim3(1), dim3(256), 0, st, (const double*)part, nb, 0.0, 1, vgoal, 31, -1.0,
                        scal);
   }
-  hipLaunchKernelGGL(k_oc_apply_flat, dim3(nblk(n)), dim3(256), 0, st, n, active, shell, rho, sens, rho_out, move,
-                     damp, rho_min, (const double*)scal);
+  hipLaunchKernelGGL(k_oc_apply_flat, dim3(nb), dim3(256), 0, st, n, (int64_t)kNoAllocChunk, active, shell, rho, sens,
+                     rho_out, move, damp, rho_min, vec, (const double*)scal);
   if (hipGetLastError() != hipSuccess) return TOS_E_HIP;
   if (g_out || steps_out) {
     double h[S_COUNT];
