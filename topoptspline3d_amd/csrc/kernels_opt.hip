@@ -147,72 +147,111 @@ __global__ __launch_bounds__(256) void k_sensitivity(LevelView L, const uint8_t*
 // ---------------------------------------------------------------------------------------
 // Filter (filterSensitivity_kernel grid/Grid.cu:4131-4216): weighted mean over the active
 // elements of a ball; offsets and weights come from a host-built table.
-// k_filter_zm<H> (table offsets within H per axis): a workgroup owns a 64 x 8 column of
-// elements and marches it along z over kFzZ planes, keeping the 2H + 1 element planes of the
+// k_filter_zm<H, TY> (table offsets within H per axis): a workgroup owns a 64 x TY column of
+// elements and marches it along z over `zc` planes, keeping the 2H + 1 element planes of the
 // current output plane, each with an H-element halo in x and y, in an LDS ring as
-// (value, 1) for active elements and (0, 0) otherwise; every thread forms two outputs per
-// plane from LDS.  Each element is loaded (64 + 2H)(8 + 2H)/512 * (kFzZ + 2H)/kFzZ times
-// (1.8 for H = 2) instead of 4.25 times with cube tiles of 64 x 4 x 4.  Both kernels walk
-// the table in its order with FP64 sums, so they give the same result (an inactive or
-// outside tap adds exactly zero to both sums).  k_filter serves larger radii.
+// (value, 1) for active elements and (0, 0) otherwise; every thread forms TY / (threads / 64)
+// outputs per plane from LDS, sharing each tap's table entry, which is uniform over the
+// workgroup and read through the scalar cache.  The next plane's loads are in flight while a
+// plane is formed; waves without an active element skip it.  Both kernels walk the table in its
+// order (dz outermost: plane d holds the taps tp.s[d] .. tp.s[d + 1]) with FP64 sums, so they
+// give the same result (an inactive or outside tap adds exactly zero to both sums).  k_filter
+// serves radii of 4.5 and more, whose ring would not fit in LDS.
+// The FP64 products bound large boxes, the number of columns small ones: `zc` (filter_planes)
+// is taken so that the fullest CU has the fewest planes to form and to fill its rings with.
+// us before (32 planes per workgroup always, the per-element kernel above H = 3; one output at
+// a time, no loads ahead) and now: 71x43x37 H = 3 314 -> 23, 128x64x64 H = 2 132 -> 20,
+// 256x128x128 H = 4 744 -> 327.
 // ---------------------------------------------------------------------------------------
-constexpr int kFzX = 64, kFzY = 8, kFzZ = 32;
+constexpr int kFzX = 64;
+struct FilterPlanes { int s[10]; };
 
-template <int H>
-__global__ __launch_bounds__(256) void k_filter_zm(LevelView L, const uint8_t* __restrict__ eact,
-                                                   const float* __restrict__ src, float* __restrict__ dst,
-                                                   const int* __restrict__ off, const double* __restrict__ wt,
-                                                   int nt) {
-  constexpr int LX = kFzX + 2 * H, LY = kFzY + 2 * H, NZ = 2 * H + 1, PL = LX * LY;
-  constexpr int NT = (2 * H + 1) * (2 * H + 1) * (2 * H + 1);  // table size bound
+template <int H, int TY>
+__global__ __launch_bounds__(TY <= 8 ? 256 : 512) void k_filter_zm(LevelView L, const uint8_t* __restrict__ eact,
+                                                                   const float* __restrict__ src,
+                                                                   float* __restrict__ dst,
+                                                                   const int* __restrict__ off,
+                                                                   const double* __restrict__ wt, FilterPlanes tp,
+                                                                   int zc) {
+  constexpr int NTH = TY <= 8 ? 256 : 512, ROWS = NTH / kFzX, R = TY / ROWS;
+  constexpr int LX = kFzX + 2 * H, LY = TY + 2 * H, NZ = 2 * H + 1, PL = LX * LY, NL = (PL + NTH - 1) / NTH;
   __shared__ float2 ring[NZ * PL];
-  __shared__ int tdz[NT], tin[NT];  // tap plane (dz + H) and offset within a plane
-  __shared__ int toffz[NT];         // LDS offset of each tap for the current output plane
-  __shared__ double twt[NT];
-  const int x0 = blockIdx.x * kFzX, y0 = blockIdx.y * kFzY, z0 = blockIdx.z * kFzZ;
-  for (int i = threadIdx.x; i < nt; i += 256) {
-    tdz[i] = off[3 * i + 2] + H;
-    tin[i] = off[3 * i] + LX * off[3 * i + 1];
-    twt[i] = wt[i];
+  const int x0 = blockIdx.x * kFzX, y0 = blockIdx.y * TY, z0 = blockIdx.z * zc;
+  const int nout = min(zc, L.ez - z0);
+  const int tx = threadIdx.x % kFzX, ty = threadIdx.x / kFzX;  // rows ty + r ROWS
+  // this thread's elements of a halo plane: offset within the element plane, -1 outside the grid
+  int po[NL];
+#pragma unroll
+  for (int j = 0; j < NL; ++j) {
+    const int i = threadIdx.x + j * NTH, gx = x0 + i % LX - H, gy = y0 + i / LX - H;
+    po[j] = (i < PL && gx >= 0 && gy >= 0 && gx < L.ex && gy < L.ey) ? (int)(L.pelem(gx, gy, 0) - L.pelem(0, 0, 0)) : -1;
   }
-  const int tx = threadIdx.x % kFzX, ty = threadIdx.x / kFzX;  // rows ty and ty + 4
-  const int nplanes = min(kFzZ, L.ez - z0) + 2 * H;
-  for (int zi = 0; zi < nplanes; ++zi) {
-    const int gz = z0 - H + zi;  // plane loaded in this step, into slot zi % NZ
-    float2* pl = ring + (zi % NZ) * PL;
-    for (int i = threadIdx.x; i < PL; i += 256) {
-      const int gx = x0 + i % LX - H, gy = y0 + i / LX - H;
-      const bool in = gx >= 0 && gy >= 0 && gz >= 0 && gx < L.ex && gy < L.ey && gz < L.ez;
-      const int64_t q = L.pelem(in ? gx : 0, in ? gy : 0, in ? gz : 0);
-      const uint8_t a = eact[q];  // both loads issue before either is used
-      const float v = src[q];
-      pl[i] = (in && a) ? make_float2(v, 1.f) : make_float2(0.f, 0.f);
+  float pv[NL];
+  uint8_t pa[NL];
+  auto fetch = [&](int gz) {
+    const bool zin = gz >= 0 && gz < L.ez;
+    const int64_t base = L.pelem(0, 0, zin ? gz : 0);
+#pragma unroll
+    for (int j = 0; j < NL; ++j) {
+      const int64_t q = base + (po[j] >= 0 ? po[j] : 0);
+      const uint8_t a = eact[q];
+      pv[j] = src[q];
+      pa[j] = (zin && po[j] >= 0) ? a : 0;
     }
-    // output plane gz - H reads the planes loaded in steps zi - 2H .. zi
-    if (zi >= 2 * H)
-      for (int i = threadIdx.x; i < nt; i += 256) toffz[i] = ((zi - 2 * H + tdz[i]) % NZ) * PL + tin[i];
+  };
+  auto put = [&](int slot) {
+#pragma unroll
+    for (int j = 0; j < NL; ++j) {
+      const int i = threadIdx.x + j * NTH;
+      if (i < PL) ring[slot * PL + i] = pa[j] ? make_float2(pv[j], 1.f) : make_float2(0.f, 0.f);
+    }
+  };
+  for (int zi = 0; zi < 2 * H; ++zi) {
+    fetch(z0 - H + zi);
+    put(zi);
+  }
+  fetch(z0 + H);
+  int s0 = 0;  // ring slot of plane z - H
+  for (int zo = 0; zo < nout; ++zo) {
+    put((s0 + 2 * H) % NZ);
     __syncthreads();
-    if (zi >= 2 * H) {
-      const float2* cen = ring + ((zi - H) % NZ) * PL;
-      for (int r = 0; r < 2; ++r) {
-        const int yy = ty + 4 * r, x = x0 + tx, y = y0 + yy;
-        if (x >= L.ex || y >= L.ey) continue;
-        const int64_t e = L.pelem(x, y, gz - H);
-        const int c = (yy + H) * LX + tx + H;
-        if (cen[c].y == 0.f) {
-          dst[e] = 0.f;
-          continue;
+    if (zo + 1 < nout) fetch(z0 + zo + 1 + H);
+    const int c = (ty + H) * LX + tx + H;
+    bool on[R], any = false;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      on[r] = ring[((s0 + H) % NZ) * PL + c + r * ROWS * LX].y != 0.f;
+      any = any || on[r];
+    }
+    double gs[R], ws[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) gs[r] = ws[r] = 0;
+    if (__any(any)) {
+#pragma unroll
+      for (int d = 0; d < NZ; ++d) {
+        int sl = s0 + d;
+        if (sl >= NZ) sl -= NZ;
+        const float2* pl = ring + sl * PL + c;
+#pragma unroll 4
+        for (int i = tp.s[d]; i < tp.s[d + 1]; ++i) {
+          const int o = off[3 * i] + LX * off[3 * i + 1];
+          const double w = wt[i];
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            const float2 sv = pl[o + r * ROWS * LX];
+            gs[r] += w * (double)sv.x;
+            ws[r] += w * (double)sv.y;
+          }
         }
-        double gs = 0, ws = 0;
-        for (int i = 0; i < nt; ++i) {
-          const float2 sv = ring[toffz[i] + c];
-          gs += twt[i] * (double)sv.x;
-          ws += twt[i] * (double)sv.y;
-        }
-        dst[e] = (float)(gs / ws);
       }
     }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int x = x0 + tx, y = y0 + ty + r * ROWS;
+      if (x < L.ex && y < L.ey) dst[L.pelem(x, y, z0 + zo)] = on[r] ? (float)(gs[r] / ws[r]) : 0.f;
+    }
     __syncthreads();
+    if (++s0 == NZ) s0 = 0;
   }
 }
 

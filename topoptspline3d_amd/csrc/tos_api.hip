@@ -3657,6 +3657,20 @@ TOS_EXPORT int tos_init_vol_sensitivity(tos_ctx* c) {
   });
 }
 
+// Planes per workgroup of k_filter_zm over `cols` columns of ez planes: a workgroup forms zc
+// planes and fills its ring with 2H + 1 before the first (about a third of a plane's time
+// each); the fewest over the 256 CUs, the larger chunk among equals.
+static int filter_planes(int cols, int ez, int H) {
+  int best = 1;
+  double cost = 0;
+  for (int zc = 1; zc <= 32; ++zc) {
+    const int64_t blocks = (int64_t)cols * ((ez + zc - 1) / zc);
+    const double t = (double)((blocks + 255) / 256) * (zc + 0.35 * (2 * H + 1));
+    if (zc == 1 || t <= cost) { cost = t; best = zc; }
+  }
+  return best;
+}
+
 TOS_EXPORT int tos_filter(tos_ctx* c, int which, double R) {
   return guard(c, [&]() {
     float* b = sens_buf(*c, which);
@@ -3684,21 +3698,33 @@ TOS_EXPORT int tos_filter(tos_ctx* c, int which, double R) {
     HIPCHK(hipMemcpyAsync(c->tmpf, b, v.NE * sizeof(float), hipMemcpyDeviceToDevice, c->stream));
     const int64_t n = (int64_t)v.ex * v.ey * v.ez;
     Prof pr(*c, P_SENS_FILTER);
-    const dim3 tg((v.ex + kFzX - 1) / kFzX, (v.ey + kFzY - 1) / kFzY, (v.ez + kFzZ - 1) / kFzZ);
     const uint8_t* ea = (const uint8_t*)c->eact;
     const float* sb = (const float*)c->tmpf;
-    if (Ri <= 1)
-      hipLaunchKernelGGL(k_filter_zm<1>, tg, dim3(256), 0, c->stream, v, ea, sb, b, (const int*)doff,
+    FilterPlanes tp{};
+    if (Ri <= 4)
+      for (int d = 0, i = 0; d <= 2 * Ri + 1; ++d) {
+        while (i < nt && off[3 * i + 2] + Ri < d) ++i;
+        tp.s[d] = i;
+      }
+#define GO(HH, TY)                                                                                             \
+  {                                                                                                            \
+    const int cols = ((v.ex + kFzX - 1) / kFzX) * ((v.ey + TY - 1) / TY), zc = filter_planes(cols, v.ez, HH);   \
+    hipLaunchKernelGGL((k_filter_zm<HH, TY>), dim3((v.ex + kFzX - 1) / kFzX, (v.ey + TY - 1) / TY,              \
+                                                   (v.ez + zc - 1) / zc),                                       \
+                       dim3(TY <= 8 ? 256 : 512), 0, c->stream, v, ea, sb, b, (const int*)doff,                 \
+                       (const double*)dwt, tp, zc);                                                             \
+  }
+    if (Ri == 0)
+      hipLaunchKernelGGL(k_filter, dim3(nblk(n)), dim3(256), 0, c->stream, v, ea, sb, b, (const int*)doff,
                          (const double*)dwt, nt);
-    else if (Ri == 2)
-      hipLaunchKernelGGL(k_filter_zm<2>, tg, dim3(256), 0, c->stream, v, ea, sb, b, (const int*)doff,
-                         (const double*)dwt, nt);
-    else if (Ri == 3)
-      hipLaunchKernelGGL(k_filter_zm<3>, tg, dim3(256), 0, c->stream, v, ea, sb, b, (const int*)doff,
-                         (const double*)dwt, nt);
+    else if (Ri == 1) GO(1, 8)
+    else if (Ri == 2) GO(2, 8)
+    else if (Ri == 3) GO(3, 8)
+    else if (Ri == 4) GO(4, 16)
     else
       hipLaunchKernelGGL(k_filter, dim3(nblk(n)), dim3(256), 0, c->stream, v, ea, sb, b, (const int*)doff,
                          (const double*)dwt, nt);
+#undef GO
     LAUNCH_CHECK();
     HIPCHK(hipStreamSynchronize(c->stream));  // the table lives in the staging buffer
     return TOS_OK;
