@@ -527,11 +527,11 @@ __global__ TOS_FINE_BOUNDS(T) void k_fine_gs_pairw(LevelView L, const int4* __re
     block_relax<T, BACKWARD>(fb[0] - s[0], fb[1] - s[1], fb[2] - s[2], D, t0, t1, t2);
   }
   if (f1 && !(cont && lane == 0)) {
-    T* dst = lane == 63 ? ub : u;  // (the next segment's lane 0 reads its start value)
+    T* dst = (ub && lane == 63) ? ub : u;  // (the next segment's lane 0 reads its start value)
     dst[p1] = v0; dst[L.NP + p1] = v1; dst[2 * L.NP + p1] = v2;
   }
   if (f2) {
-    T* dst = (lane == 0 || lane == 62) ? ub : u;
+    T* dst = (ub && (lane == 0 || lane == 62)) ? ub : u;
     dst[p1 + 1] = t0; dst[L.NP + p1 + 1] = t1; dst[2 * L.NP + p1 + 1] = t2;
   }
   if constexpr (DOTS) {  // each node once: where it is written (to u or to ub)
@@ -741,6 +741,18 @@ __device__ __forceinline__ T ld_row(const T* row, uint32_t i) {
     return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, i * 4u, 0, 0));
 }
 
+// the same value where the whole stencil is below 4 GiB: one resource for all rows, the row's
+// byte offset in a scalar register
+template <class T>
+__device__ __forceinline__ T ld_at(const T* base, uint32_t row_bytes, uint32_t i) {
+  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), (short)0, -1,
+                                                                      0x00020000);
+  if constexpr (sizeof(T) == 8)
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, i * 8u, row_bytes, 0));
+  else
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, i * 4u, row_bytes, 0));
+}
+
 template <class T>
 struct StFull {  // T entries at (9k + e) NS + s
   const T* __restrict__ p;
@@ -748,6 +760,9 @@ struct StFull {  // T entries at (9k + e) NS + s
   static constexpr bool kScaled = false;
   __device__ __forceinline__ T get(int64_t s, int k, int e) const {
     return ld_row(p + (int64_t)(k * 9 + e) * NS, (uint32_t)s);
+  }
+  __device__ __forceinline__ T at(int64_t s, int k, int e) const {  // get() of a stencil below 4 GiB
+    return ld_at(p, (uint32_t)(k * 9 + e) * (uint32_t)NS * (uint32_t)sizeof(T), (uint32_t)s);
   }
   __device__ __forceinline__ T scale(int64_t) const { return T(1); }
 };
@@ -773,6 +788,12 @@ struct StHalf {
     const int w = e < 8 ? 4 * k + (e >> 1) : 108 + (k >> 1);
     const int hi = e < 8 ? (e & 1) : (k & 1);
     const uint32_t v = ld_row(p + (int64_t)w * NS, (uint32_t)s);
+    return half_bits(hi ? (v >> 16) : (v & 0xffffu));
+  }
+  __device__ __forceinline__ float at(int64_t s, int k, int e) const {
+    const int w = e < 8 ? 4 * k + (e >> 1) : 108 + (k >> 1);
+    const int hi = e < 8 ? (e & 1) : (k & 1);
+    const uint32_t v = ld_at(p, (uint32_t)w * (uint32_t)NS * 4u, (uint32_t)s);
     return half_bits(hi ? (v >> 16) : (v & 0xffffu));
   }
   __device__ __forceinline__ float scale(int64_t s) const { return msc[s]; }
@@ -973,6 +994,195 @@ __global__ __launch_bounds__(256) void k_st_gs_pairw(LevelView L, const int4* __
   if (f2) {
     T* dst = (ub && (lane == 0 || lane == 62)) ? ub : u;
     dst[pa + 1] = t0; dst[L.NP + pa + 1] = t1; dst[2 * L.NP + pa + 1] = t2;
+  }
+}
+
+// ---------------------------------------------------------------------------------------
+// Stored-stencil kernels of the levels with few rows (gs_split, apply_split in the host code).  A pass
+// over such a level has too few waves to hide a node's loads behind other nodes', so its time
+// is the chain of the loads that one thread issues.  Here several waves share a node: each sums
+// the blocks of its neighbour rows (dy, dz) = (r % 3 - 1, r / 3 - 1), all loads of a row in
+// flight together, and leaves the sum in LDS; the wave that has the centre row adds the others'
+// to its own and finishes the node.
+// ---------------------------------------------------------------------------------------
+
+// loads of stencil row r (blocks 3r .. 3r + 2) at `slot`, and its product with the columns
+// c[J], c[J + 1], c[J + 2]; kept apart so that all loads of a row are in flight together
+template <class T, class ST>
+__device__ __forceinline__ void st_row_load(const ST& st, int64_t slot, int r, T (&A)[3][9]) {
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+#pragma unroll
+    for (int e = 0; e < 9; ++e) A[j][e] = st.at(slot, 3 * r + j, e);
+}
+template <class T, int J>
+__device__ __forceinline__ void st_row_add(const T (&A)[3][9], const T (&c)[4][3], T (&s)[3]) {
+  T t[3] = {0, 0, 0};
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+#pragma unroll
+    for (int e = 0; e < 9; ++e) t[e / 3] = fma(A[j][e], c[J + j][e % 3], t[e / 3]);
+#pragma unroll
+  for (int e = 0; e < 3; ++e) s[e] += t[e];
+}
+
+// k_st_gs_pairw on such a level (the same segments, each a whole grid row, so no node is
+// deferred): one workgroup per segment.  Only the centre row holds nodes of this pass, so the
+// other rows' sums are those of both colours, and only the centre wave waits for the first
+// colour's values.  ZERO: the first sweep from zero, where only rows of earlier classes hold
+// values.  Three waves, one per node plane: nine were no faster with FP16 and FP32 stencils and
+// slower with FP64, whose loads of a row they have no registers for (28 against 19 us a pass at
+// 420 rows of 80 nodes).
+template <class T, bool BACKWARD, bool ZERO, class ST>
+__global__ __launch_bounds__(192) void k_st_gs_split(LevelView L, const int4* __restrict__ seg,
+                                                         const int* __restrict__ slotmap, ST st, T* __restrict__ u,
+                                                         const T* __restrict__ f, int cls) {
+  __shared__ T part[2][6][64];
+  const int4 S = seg[xcd_block()];
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int xs = (S.y & 0x7fff) - 1, xe = ((S.y >> 15) & 0x7fff) - 1;
+  const int x1 = xs + 2 * lane;
+  const bool live = x1 <= xe + 1;
+  const int xa = live ? x1 : xe + 1;  // loads from addresses clamped into the row
+  const int64_t pa = (int64_t)S.x + (xa - xs);
+  const int sl1 = slotmap[pa], sl2 = slotmap[pa + 1];
+  const bool f1 = live && sl1 >= 0;
+  const bool f2 = live && lane < 63 && x1 + 1 <= xe && sl2 >= 0;
+  const int s1 = f1 ? sl1 : 0, s2 = f2 ? sl2 : 0;
+  const auto dy = [&](int r) { return r % 3 - 1; };
+  const auto dz = [&](int r) { return r / 3 - 1; };
+  // does row r hold values (from zero: this class's and later ones' do not yet)
+  const auto holds = [&](int r) { return !ZERO || (cls ^ ((dy(r) & 1) | ((dz(r) & 1) << 1))) < cls; };
+  const auto load = [&](int r, T (&c)[4][3]) {  // columns x1 - 1 .. x1 + 2 of row r
+    const int64_t q = pa + (int64_t)L.NX * (dy(r) + (int64_t)L.NY * dz(r));
+    const int64_t qc[4] = {xa >= 0 ? q - 1 : q, q, q + 1, xa + 2 <= xe + 1 ? q + 2 : q};
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int e = 0; e < 3; ++e) c[j][e] = u[e * L.NP + qc[j]];
+  };
+  T a[3] = {0, 0, 0}, b[3] = {0, 0, 0};
+  const auto add = [&](int i) {
+    const int r = 3 * wv + i;
+    if (holds(r)) {
+      T c[4][3];
+      T A1[3][9], A2[3][9];
+      load(r, c);
+      st_row_load(st, s1, r, A1);
+      st_row_load(st, s2, r, A2);
+      TOS_LOADS_DONE();
+      st_row_add<T, 0>(A1, c, a);
+      st_row_add<T, 1>(A2, c, b);
+    }
+  };
+  if (wv != 1) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) add(i);
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {
+      part[wv >> 1][e][lane] = a[e];
+      part[wv >> 1][3 + e][lane] = b[e];
+    }
+    __syncthreads();
+    return;
+  }
+  T c[4][3] = {};  // the centre row (from zero: nothing there yet)
+  if (!ZERO) load(4, c);
+  T A1[3][9], A2[3][9];
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+#pragma unroll
+    for (int e = 0; e < 9; ++e) {
+      A1[j][e] = (ZERO && j != 1) ? T(0) : st.at(s1, 12 + j, e);
+      A2[j][e] = st.at(s2, 12 + j, e);
+    }
+  T fa[3], fb[3];
+#pragma unroll
+  for (int e = 0; e < 3; ++e) {
+    fa[e] = f[e * L.NP + pa];
+    fb[e] = f[e * L.NP + pa + 1];
+  }
+  T i1 = 1, i2 = 1;  // a scaled stencil's equations are solved in the scaled form (see st_relax)
+  if constexpr (ST::kScaled) {
+    i1 = T(1) / st.scale(s1);
+    i2 = T(1) / st.scale(s2);
+  }
+  add(0);
+  add(2);
+  if (!ZERO) {
+#pragma unroll
+    for (int j = 0; j < 3; j += 2)
+#pragma unroll
+      for (int e = 0; e < 9; ++e) a[e / 3] = fma(A1[j][e], c[j][e % 3], a[e / 3]);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < 3; ++e) {
+    a[e] += part[0][e][lane] + part[1][e][lane];
+    b[e] += part[0][3 + e][lane] + part[1][3 + e][lane];
+  }
+  T v[3] = {c[1][0], c[1][1], c[1][2]};
+  if (f1) block_relax<T, BACKWARD>(fma(fa[0], i1, -a[0]), fma(fa[1], i1, -a[1]), fma(fa[2], i1, -a[2]), A1[1], v[0],
+                                  v[1], v[2]);
+  T w[3];
+#pragma unroll
+  for (int e = 0; e < 3; ++e) w[e] = __shfl_down(v[e], 1, 64);  // the next lane's first-colour node
+#pragma unroll
+  for (int e = 0; e < 9; ++e) b[e / 3] = fma(A2[0][e], v[e % 3], b[e / 3]);
+#pragma unroll
+  for (int e = 0; e < 9; ++e) b[e / 3] = fma(A2[2][e], w[e % 3], b[e / 3]);
+  T t[3] = {c[2][0], c[2][1], c[2][2]};
+  if (f2) block_relax<T, BACKWARD>(fma(fb[0], i2, -b[0]), fma(fb[1], i2, -b[1]), fma(fb[2], i2, -b[2]), A2[1], t[0],
+                                  t[1], t[2]);
+#pragma unroll
+  for (int e = 0; e < 3; ++e) {
+    if (f1) u[e * L.NP + pa] = v[e];
+    if (f2) u[e * L.NP + pa + 1] = t[e];
+  }
+}
+
+// k_st_apply on such a level, one workgroup per chunk of the colour-ordered list, a wave per
+// neighbour row.
+template <class T, int MODE, class ST>
+__global__ __launch_bounds__(576) void k_st_apply_split(LevelView L, const int4* __restrict__ cl, ST st,
+                                                        const T* __restrict__ u, const T* __restrict__ f,
+                                                        T* __restrict__ y) {
+  __shared__ T part[8][3][64];
+  const int ch = (int)xcd_block();
+  const int r = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int4 C = cl[ch];
+  const bool on = lane < (C.y >> 16);
+  const int64_t p = (int64_t)C.x + 2 * (on ? lane : 0), slot = (int64_t)ch * 64 + lane;
+  const int64_t q = p + (int64_t)L.NX * (r % 3 - 1 + (int64_t)L.NY * (r / 3 - 1));
+  T c[4][3], s[3] = {0, 0, 0};
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+#pragma unroll
+    for (int e = 0; e < 3; ++e) c[j][e] = u[e * L.NP + q + j - 1];
+  T A[3][9];
+  st_row_load(st, slot, r, A);
+  TOS_LOADS_DONE();
+  st_row_add<T, 0>(A, c, s);
+  if (r != 4) {
+#pragma unroll
+    for (int e = 0; e < 3; ++e) part[r < 4 ? r : r - 1][e][lane] = s[e];
+    __syncthreads();
+    return;
+  }
+  T fp[3] = {0, 0, 0}, m = 1;
+  if (MODE == 1) {
+#pragma unroll
+    for (int e = 0; e < 3; ++e) fp[e] = f[e * L.NP + p];
+  }
+  if constexpr (ST::kScaled) m = st.scale(slot);
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < 3; ++e) {
+    T t[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) t[i] = part[i][e][lane];
+    const T v = s[e] + (((t[0] + t[7]) + (t[1] + t[6])) + ((t[2] + t[5]) + (t[3] + t[4])));  // opposite rows together
+    if (on) y[e * L.NP + p] = MODE == 1 ? fma(-v, m, fp[e]) : v * m;
   }
 }
 

@@ -853,7 +853,8 @@ void gs_sweep_pairs(Ctx& c, T* u, const T* f, bool backward, bool from_zero) {
 void gs_sweep_pairw(Ctx& c, float* u, const float* f, bool backward, bool from_zero) {
   Level& L = c.L[0];
   const LevelView& v = L.v;
-  if (!L.ub32) L.ub32 = dalloc<float>(c, 3 * (size_t)v.NP);
+  if (!L.pair_single && !L.ub32) L.ub32 = dalloc<float>(c, 3 * (size_t)v.NP);
+  float* ub = L.pair_single ? nullptr : L.ub32;  // rows of one segment: no deferred nodes
   const int P = backward ? 1 : 0;
   // the FCG's z.r and z.q from this sweep's final values (one sum per wave and pass)
   // (c.gsdots is sized by the solve before any capture: one zr and one zq per segment)
@@ -871,17 +872,17 @@ void gs_sweep_pairw(Ctx& c, float* u, const float* f, bool backward, bool from_z
     const uint8_t* fr = L.fre;
     if (dots) {
       hipLaunchKernelGGL((k_fine_gs_pairw<float, true, -1, -1, true>), g, b, 0, c.stream, v, sg, n, fr, c.w32,
-                         c.Kc32, u, f, L.ub32, c.dots_q, c.gsdots + doff, nd);
+                         c.Kc32, u, f, ub, c.dots_q, c.gsdots + doff, nd);
       doff += n;
     } else if (backward) {
       hipLaunchKernelGGL((k_fine_gs_pairw<float, true, -1, -1>), g, b, 0, c.stream, v, sg, n, fr, c.w32, c.Kc32, u, f,
-                         L.ub32, (const float*)nullptr, (double*)nullptr, (int64_t)0);
+                         ub, (const float*)nullptr, (double*)nullptr, (int64_t)0);
     } else if (!from_zero) {
       hipLaunchKernelGGL((k_fine_gs_pairw<float, false, -1, -1>), g, b, 0, c.stream, v, sg, n, fr, c.w32, c.Kc32, u,
-                         f, L.ub32, (const float*)nullptr, (double*)nullptr, (int64_t)0);
+                         f, ub, (const float*)nullptr, (double*)nullptr, (int64_t)0);
     } else {
 #define GO(A) hipLaunchKernelGGL((k_fine_gs_pairw<float, false, A, A + 1>), g, b, 0, c.stream, v, sg, n, fr, c.w32, \
-                                 c.Kc32, u, f, L.ub32, (const float*)nullptr, (double*)nullptr, (int64_t)0)
+                                 c.Kc32, u, f, ub, (const float*)nullptr, (double*)nullptr, (int64_t)0)
       switch (cls) {
         case 0: GO(0); break;
         case 1: GO(2); break;
@@ -890,12 +891,27 @@ void gs_sweep_pairw(Ctx& c, float* u, const float* f, bool backward, bool from_z
       }
 #undef GO
     }
-    hipLaunchKernelGGL((k_fine_pairw_copy<float>), dim3(nblk(3 * (int64_t)n)), dim3(256), 0, c.stream, v, sg, n, fr,
-                       (const float*)L.ub32, u);
+    if (ub)
+      hipLaunchKernelGGL((k_fine_pairw_copy<float>), dim3(nblk(3 * (int64_t)n)), dim3(256), 0, c.stream, v, sg, n, fr,
+                         (const float*)ub, u);
   }
   if (dots) c.dots_done = true;
   LAUNCH_CHECK();
 }
+
+// Stored-stencil levels whose passes are short of waves take the kernels with several waves per
+// row (k_st_gs_split, k_st_apply_split), whatever the sweep mode and the cycle's precision.
+// Every row has to be one segment (at most 126 nodes), so that no node is deferred, and the
+// stencil below 4 GiB.  us a sweep pass / a residual, one wave and several: FP16 at 250 rows
+// 7.8 -> 5.7 / 7.5 -> 4.6, at 900 rows 12 against 13 / 9.3 (550 chunks) against 6.7 but 38
+// against 50 at 1900; FP32 at 290 rows 13.5 -> 9.0 / 6.8 -> 4.5; FP64 at 420 rows 2 x 17 (one
+// colour a pass) -> 19, at 110 rows 2 x 11.5 -> 7.5 / 14.5 -> 7.8, at 880 chunks 16 against 23.
+constexpr int kSplitBelow = 512;
+inline bool small_stencil(const Level& L) { return L.NS * 243 * (int64_t)sizeof(double) < (int64_t)1 << 32; }
+inline bool gs_split(const Level& L) {
+  return L.pair_ok && L.pair_single && L.n_segw[0][0] < kSplitBelow && small_stencil(L);
+}
+inline bool apply_split(const Level& L) { return L.n_col < kSplitBelow; }
 
 // Stored-stencil level sweep in four in-wave two-colour passes (k_st_gs_pairw), each
 // followed by the copy of its deferred nodes when rows span several segments; same class
@@ -943,10 +959,34 @@ void gs_sweep_st_pairw(Ctx& c, int l, T* u, const T* f, bool backward, bool from
   LAUNCH_CHECK();
 }
 
+// Sweep of a level with few rows, two colours per pass and three waves per row
+template <class T>
+void gs_sweep_st_split(Ctx& c, int l, T* u, const T* f, bool backward, bool from_zero) {
+  Level& L = c.L[l];
+  for (int i = 0; i < 4; ++i) {
+    const int cls = backward ? 3 - i : i;
+    const int n = L.n_segw[cls][backward ? 1 : 0];
+    if (!n) continue;
+    Prof pr(c, sizeof(T) == 8 ? P_ST_GS64 : (l == 1 ? P_ST_GS32_L1 : P_ST_GS32));
+    const int4* sg = L.segw[cls][backward ? 1 : 0];
+    st_dispatch<T>(c, L, [&](auto st) {
+      using ST = decltype(st);
+      auto k = backward ? &k_st_gs_split<T, true, false, ST>
+                        : (from_zero ? &k_st_gs_split<T, false, true, ST> : &k_st_gs_split<T, false, false, ST>);
+      hipLaunchKernelGGL(k, dim3(n), dim3(192), 0, c.stream, L.v, sg, (const int*)L.slot, st, u, f, cls);
+    });
+  }
+  LAUNCH_CHECK();
+}
+
 template <class T>
 void gs_sweep(Ctx& c, int l, T* u, const T* f, bool backward, bool from_zero = false) {
   Level& L = c.L[l];
   const LevelView& v = L.v;
+  if (l > 0 && gs_split(L)) {
+    gs_sweep_st_split<T>(c, l, u, f, backward, from_zero);
+    return;
+  }
   if constexpr (std::is_same<T, float>::value) {
     if (l == 0 && c.sweep_mode == 3) {
       gs_sweep_pairw(c, u, f, backward, from_zero);
@@ -1029,6 +1069,11 @@ void apply_level(Ctx& c, int l, const T* u, const T* f, T* y, double* partial = 
     }
   } else if (L.n_col) {
     st_dispatch<T>(c, L, [&](auto st) {
+      if (apply_split(L)) {
+        hipLaunchKernelGGL((k_st_apply_split<T, MODE, decltype(st)>), dim3(L.n_col), dim3(576), 0, c.stream, L.v,
+                           (const int4*)L.cl_col, st, u, f, y);
+        return;
+      }
       hipLaunchKernelGGL((k_st_apply<T, MODE, decltype(st)>), dim3(cblk(L.n_col)), dim3(256), 0, c.stream, L.v,
                          (const int4*)L.cl_col, L.n_col, st, u, f, y);
     });
