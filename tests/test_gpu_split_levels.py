@@ -1,7 +1,8 @@
 """V-cycles whose stencil levels take several waves per row, against the FP64 oracle: rows of
 one pair and of the largest single segment (126 free nodes, 252 elements on the fine level;
 with 256 the level's rows are two segments and it keeps the one-wave kernels), odd sizes, voids
-that break rows, supports that start rows at x = 0 and at x = 1.  FP64 cycles agree to rounding
+that break rows, supports that start rows at x = 0 and at x = 1 (the long boxes stand on z = 0:
+as cantilevers their coarsest solve alone, of condition 1e7, differs from the oracle's by 3e-9).  FP64 cycles agree to rounding
 (relative 1e-11 over a few thousand operations of condition up to 1e4); FP32 ones to 2e-4 and
 FP16 stencils to 1e-2 as in the general V-cycle test."""
 import numpy as np
@@ -15,7 +16,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dims,void,zsup", [((9, 9, 40), 0.0, False), ((10, 24, 11), 0.3, True),
-                                            ((252, 10, 9), 0.1, False), ((256, 9, 10), 0.1, True),
+                                            ((252, 10, 9), 0.1, True), ((256, 9, 10), 0.1, True),
                                             ((37, 41, 23), 0.25, False), ((64, 50, 33), 0.0, True)])
 def test_vcycles_match_oracle(dims, void, zsup):
     from topoptspline3d_amd.backend import gpu_available, hip_api

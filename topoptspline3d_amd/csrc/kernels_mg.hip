@@ -1582,7 +1582,11 @@ __global__ __launch_bounds__(256) void k_cast_nodes(const int4* __restrict__ cl,
 // output in the compact layout.
 // First coarse level: the coarse element matrices are sum over active children of
 // rho^p P_c^T Ke P_c (8 precomputed 24x24 products Mc), evaluated with the eliminated
-// rows/columns when a child touches a non-free fine node (allfree[e] = 0)
+// rows/columns when a child touches a non-free fine node: fpat[e] = 1 all its nodes are free,
+// 2 + q the q-th product of Mp (one per child position and set of free nodes that the fine
+// level has, at most kGalPatterns), 0 any other, summed node by node.  A row of a box touches
+// its support plane once, so every wave of the launch has such a child; summed node by node
+// they took most of it (us, before and now: 743 -> 147 at 128x64x64, 233 -> 43 at 24x12x12)
 // (restrict_stencil_nondyadic_OTFA_WS_kernel grid/Grid.cu:1112-1225 computes the same
 // triple product per coarse node directly from the fine densities).
 // ---------------------------------------------------------------------------------------
@@ -1636,8 +1640,9 @@ __device__ __noinline__ GalPair gal_row_partial(const LevelView F, const uint8_t
 template <int AX>
 __device__ __forceinline__ void gal_elem_row(const LevelView& F, const LevelView& C, int X, int Y, int Z, int ay,
                                              int az, int jy, int jz, const uint8_t* __restrict__ ffre,
-                                             const uint8_t* __restrict__ fallfree, const double* __restrict__ w,
+                                             const uint8_t* __restrict__ fpat, const double* __restrict__ w,
                                              const double* __restrict__ Ke, const double* __restrict__ Mc,
+                                             const double* __restrict__ Mp,
                                              double (&acc)[3][9]) {
   const int Ex = X - 1 + AX, Ey = Y - 1 + ay, Ez = Z - 1 + az;
   if (Ex < 0 || Ey < 0 || Ez < 0 || Ex >= C.ex || Ey >= C.ey || Ez >= C.ez) return;
@@ -1651,14 +1656,14 @@ __device__ __forceinline__ void gal_elem_row(const LevelView& F, const LevelView
     const bool in = fx < F.ex && fy < F.ey && fz < F.ez;
     const int64_t fe = F.pelem(in ? fx : 0, in ? fy : 0, in ? fz : 0);
     wc[ch] = w[fe];
-    af[ch] = fallfree[fe];
+    af[ch] = fpat[fe];
     if (!in) wc[ch] = 0;
   }
 #pragma unroll
   for (int ch = 0; ch < 8; ++ch) {
     const double we = wc[ch];
     if (we == 0) continue;
-    if (af[ch]) {
+    if (af[ch] == 1) {
       const double* m0 = Mc + ch * 576 + (3 * mI) * 24 + 3 * (2 * jy + 4 * jz);
 #pragma unroll
       for (int jx = 0; jx < 2; ++jx) {
@@ -1668,7 +1673,13 @@ __device__ __forceinline__ void gal_elem_row(const LevelView& F, const LevelView
 #pragma unroll
           for (int c = 0; c < 3; ++c) acc[jx + AX][r * 3 + c] += we * m[r * 24 + c];
       }
-    } else {  // a fine node of the child is eliminated: rare, out of line
+    } else if (af[ch]) {  // (the lane's own product)
+      const double* m0 = Mp + (af[ch] - 2) * 576 + (3 * mI) * 24 + 3 * (2 * jy + 4 * jz);
+#pragma unroll
+      for (int jx = 0; jx < 2; ++jx)
+#pragma unroll
+        for (int e = 0; e < 9; ++e) acc[jx + AX][e] += we * m0[3 * jx + (e / 3) * 24 + e % 3];
+    } else {  // out of line
       const int fx = 2 * Ex + (ch & 1), fy = 2 * Ey + ((ch >> 1) & 1), fz = 2 * Ez + (ch >> 2);
       const GalPair t = gal_row_partial(F, ffre, Ke, fx, fy, fz, ch, mI, jy, jz, we);
 #pragma unroll
@@ -1681,11 +1692,12 @@ __device__ __forceinline__ void gal_elem_row(const LevelView& F, const LevelView
 
 __global__ __launch_bounds__(256) void k_galerkin_first_row(LevelView F, LevelView C, const int4* __restrict__ clc,
                                                             int nch, const uint8_t* __restrict__ ffre,
-                                                            const uint8_t* __restrict__ fallfree,
+                                                            const uint8_t* __restrict__ fpat,
                                                             const uint8_t* __restrict__ cfre,
                                                             const double* __restrict__ w,
                                                             const double* __restrict__ Ke,
-                                                            const double* __restrict__ Mc, double* __restrict__ st,
+                                                            const double* __restrict__ Mc,
+                                                            const double* __restrict__ Mp, double* __restrict__ st,
                                                             float* __restrict__ st32, int64_t NS) {
   NodeRef nr;
   if (!chunk_node(clc, nch, 2, nr)) return;
@@ -1702,8 +1714,8 @@ __global__ __launch_bounds__(256) void k_galerkin_first_row(LevelView F, LevelVi
     for (int ay = 0; ay < 2; ++ay) {
       const int jy = 1 + dy - ay;
       if (jy < 0 || jy > 1) continue;
-      gal_elem_row<0>(F, C, X, Y, Z, ay, az, jy, jz, ffre, fallfree, w, Ke, Mc, acc);
-      gal_elem_row<1>(F, C, X, Y, Z, ay, az, jy, jz, ffre, fallfree, w, Ke, Mc, acc);
+      gal_elem_row<0>(F, C, X, Y, Z, ay, az, jy, jz, ffre, fpat, w, Ke, Mc, Mp, acc);
+      gal_elem_row<1>(F, C, X, Y, Z, ay, az, jy, jz, ffre, fpat, w, Ke, Mc, Mp, acc);
     }
   }
 #pragma unroll

@@ -140,28 +140,32 @@ double pweight_h(int c, int i, int m) {
   return w;
 }
 
-// Mc[c] = P_c^T Ke P_c for the 8 child positions c of a fine element in its coarse element
+// M = P_c^T Ke P_c for child position c of a fine element in its coarse element, with the rows
+// and columns of the element's nodes outside `mask` left out
+void child_product(const double* Ke, int c, unsigned mask, double* M) {
+  double P[8][8];
+  for (int i = 0; i < 8; ++i)
+    for (int m = 0; m < 8; ++m) P[i][m] = (mask >> i) & 1 ? pweight_h(c, i, m) : 0.0;
+  double T[24][24];
+  for (int i = 0; i < 24; ++i)
+    for (int n = 0; n < 8; ++n)
+      for (int s = 0; s < 3; ++s) {
+        double acc = 0;
+        for (int j = 0; j < 8; ++j) acc += Ke[i * 24 + 3 * j + s] * P[j][n];
+        T[i][3 * n + s] = acc;
+      }
+  for (int m = 0; m < 8; ++m)
+    for (int r = 0; r < 3; ++r)
+      for (int col = 0; col < 24; ++col) {
+        double acc = 0;
+        for (int i = 0; i < 8; ++i) acc += P[i][m] * T[3 * i + r][col];
+        M[(3 * m + r) * 24 + col] = acc;
+      }
+}
+
+// Mc[c]: the products of whole elements
 void child_products(const double* Ke, double* Mc) {
-  for (int c = 0; c < 8; ++c) {
-    double P[8][8];
-    for (int i = 0; i < 8; ++i)
-      for (int m = 0; m < 8; ++m) P[i][m] = pweight_h(c, i, m);
-    static thread_local double T[24][24];
-    for (int i = 0; i < 24; ++i)
-      for (int n = 0; n < 8; ++n)
-        for (int s = 0; s < 3; ++s) {
-          double acc = 0;
-          for (int j = 0; j < 8; ++j) acc += Ke[i * 24 + 3 * j + s] * P[j][n];
-          T[i][3 * n + s] = acc;
-        }
-    for (int m = 0; m < 8; ++m)
-      for (int r = 0; r < 3; ++r)
-        for (int col = 0; col < 24; ++col) {
-          double acc = 0;
-          for (int i = 0; i < 8; ++i) acc += P[i][m] * T[3 * i + r][col];
-          Mc[c * 576 + (3 * m + r) * 24 + col] = acc;
-        }
-  }
+  for (int c = 0; c < 8; ++c) child_product(Ke, c, 255, Mc + c * 576);
 }
 
 // The same for a factor-4 coarsening (skip-layer): the 64 fine elements of a coarse
@@ -2752,20 +2756,29 @@ TOS_EXPORT int tos_ctx_create(const tos_grid_desc* d, tos_ctx** out) {
     auto pe = pad_elems(v0, c->h_solid.data());
     upload(c->stream, c->eact, pe.data(), v0.NE);
     {
-      // active elements whose 8 nodes are all free (Galerkin fast path)
+      // free nodes of each active element, as the pattern of its child product (gal_pat)
       std::vector<uint8_t> af(v0.NE, 0);
       const Level& L0h = c->L[0];
+      std::vector<int> number(8 << 8, -1);
       for (int z = 0; z < v0.ez; ++z)
         for (int y = 0; y < v0.ey; ++y)
           for (int x = 0; x < v0.ex; ++x) {
             if (!pe[v0.pelem(x, y, z)]) continue;
-            bool all = true;
-            for (int j = 0; j < 8 && all; ++j)
-              all = L0h.h_free[(x + (j & 1)) + (size_t)v0.nx * ((y + ((j >> 1) & 1)) + (size_t)v0.ny * (z + (j >> 2)))];
-            af[v0.pelem(x, y, z)] = all;
+            int mask = 0;
+            for (int j = 0; j < 8; ++j)
+              mask |= (L0h.h_free[(x + (j & 1)) + (size_t)v0.nx * ((y + ((j >> 1) & 1)) + (size_t)v0.ny * (z + (j >> 2)))] ? 1 : 0) << j;
+            uint8_t& a = af[v0.pelem(x, y, z)];
+            if (mask == 255) { a = 1; continue; }
+            const int key = (x & 1) | ((y & 1) << 1) | ((z & 1) << 2) | (mask << 3);
+            if (number[key] < 0 && (int)c->gal_pats.size() < kGalPatterns) {
+              number[key] = (int)c->gal_pats.size();
+              c->gal_pats.push_back(key);
+            }
+            if (number[key] >= 0) a = (uint8_t)(2 + number[key]);
           }
-      c->allfree = dalloc<uint8_t>(*c, v0.NE);
-      upload(c->stream, c->allfree, af.data(), v0.NE);
+      c->gal_pat = dalloc<uint8_t>(*c, v0.NE);
+      upload(c->stream, c->gal_pat, af.data(), v0.NE);
+      c->Mp64 = dalloc<double>(*c, 576 * std::max<size_t>(1, c->gal_pats.size()));
       if (c->skip) {
         // which nodes of each active fine element are supported (the penalty of the
         // skip-layer Galerkin operator)
@@ -2924,6 +2937,12 @@ TOS_EXPORT int tos_set_material(tos_ctx* c, double E, double nu, double p, doubl
     upload(c->stream, c->Kc64, kc, sizeof(kc));
     upload(c->stream, c->Kc32, kc32, sizeof(kc32));
     upload(c->stream, c->Mc64, c->h_Mc, sizeof(c->h_Mc));
+    if (!c->gal_pats.empty()) {
+      std::vector<double> mp(576 * c->gal_pats.size());
+      for (size_t q = 0; q < c->gal_pats.size(); ++q)
+        child_product(c->h_Ke, c->gal_pats[q] & 7, (unsigned)c->gal_pats[q] >> 3, mp.data() + 576 * q);
+      upload(c->stream, c->Mp64, mp.data(), mp.size() * sizeof(double));
+    }
     if (c->skip) {
       std::vector<double> m4(64 * 576);
       child_products4(c->h_Ke, m4.data());
@@ -3085,9 +3104,9 @@ void galerkin_levels(Ctx& c, bool copy32) {
                          (!d64 || copy32) ? C.st32 : (float*)nullptr, C.NS);
     else if (l == 1)
       hipLaunchKernelGGL(k_galerkin_first_row, dim3(cblk(C.n_col), 9), dim3(256), 0, c.stream, F.v, C.v,
-                         (const int4*)C.cl_col, C.n_col, (const uint8_t*)F.fre, (const uint8_t*)c.allfree,
+                         (const int4*)C.cl_col, C.n_col, (const uint8_t*)F.fre, (const uint8_t*)c.gal_pat,
                          (const uint8_t*)C.fre, (const double*)c.w64, (const double*)c.Ke64,
-                         (const double*)c.Mc64, d64 ? C.st64 : (double*)nullptr,
+                         (const double*)c.Mc64, (const double*)c.Mp64, d64 ? C.st64 : (double*)nullptr,
                          (!d64 || copy32) ? C.st32 : (float*)nullptr, C.NS);
     else
       galerkin_by_axes<TS>(c, F, C, copy32);

@@ -145,7 +145,9 @@ struct Ctx {
   int64_t n_active = 0;
   // fine-level element data (padded element layout)
   uint8_t* eact = nullptr;
-  uint8_t* allfree = nullptr;   // active element whose 8 nodes are all free
+  uint8_t* gal_pat = nullptr;   // per padded fine element: 1 all 8 nodes free, 2 + q pattern q, 0 other
+  std::vector<int> gal_pats;    // patterns: child position | free-node mask << 3, at most kGalPatterns
+  double* Mp64 = nullptr;       // 576 per pattern: its child product
   uint8_t* shell = nullptr;
   float* rho = nullptr;
   float* rho_pre = nullptr;
@@ -304,6 +306,7 @@ struct Ctx {
                                 // a captured graph from an older epoch is destroyed, not replayed
 };
 
+constexpr int kGalPatterns = 254;  // (their numbers fit a byte beside 0 and 1; 1.2 MB of products)
 constexpr int kRedBlocks = 1024;  // fixed partial count -> deterministic reductions
 
 }  // namespace tos
