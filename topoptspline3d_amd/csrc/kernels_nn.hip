@@ -4,8 +4,8 @@
 // Tensors are channel-last BF16 ("x[v * cs + co + c]", v = x + X*(y + Y*z) + b*V) with a
 // channel stride `cs` and offset `co`, so a decoder's skip-concatenation buffer is written
 // in place by the encoder.  Convolutions are implicit GEMMs on MFMA
-// (v_mfma_f32_16x16x32_bf16, FP32 accumulation): one wave computes 16 consecutive output
-// voxels of a row (A rows) x all output channels (B columns, NOUT/16 tiles); the K
+// (v_mfma_f32_16x16x32_bf16, FP32 accumulation): one wave computes tiles of 16 consecutive
+// output voxels (A rows) x 16 output channels (B columns); the K
 // dimension runs over (tap, input channel) with tap = (dx+1) + 3(dy+1) + 9(dz+1), so one
 // lane's 8 consecutive K values are 8 channels of one tap (one 16-byte load).
 //   MODE 0 forward, stride 1:   y[o] = sum_t W_t x[o + d_t]
@@ -32,6 +32,33 @@ struct NGrid {
   int X, Y, Z;
 };
 
+// quotient of v < 2^31 by n as a multiplication: with 2^(s-1) < n <= 2^s and
+// m = floor(2^(31+s) / n) + 1, m n exceeds 2^(31+s) by at most 2^s, so v m / 2^(31+s) is above
+// v / n by less than 1 / n
+struct DivBy {
+  uint32_t n, m, s;
+};
+inline DivBy div_by(int n) {
+  DivBy d{(uint32_t)n, 0, 0};
+  while ((1ull << d.s) < d.n) ++d.s;
+  d.m = (uint32_t)((1ull << (31 + d.s)) / d.n + 1);
+  return d;
+}
+// v = q n + r
+__device__ __forceinline__ uint32_t div_step(const DivBy& d, uint32_t v, int& r) {
+  const uint32_t q = (uint32_t)(((uint64_t)v * d.m) >> (31 + d.s));
+  r = (int)(v - q * d.n);
+  return q;
+}
+struct VoxDiv {
+  DivBy x, y, z;
+};
+inline VoxDiv vox_div(const NGrid& g) { return VoxDiv{div_by(g.X), div_by(g.Y), div_by(g.Z)}; }
+// batch index and coordinates of voxel v of a grid
+__device__ __forceinline__ int vox_at(const VoxDiv& d, uint32_t v, int& x, int& y, int& z) {
+  return (int)div_step(d.z, div_step(d.y, div_step(d.x, v, x), y), z);
+}
+
 __device__ __forceinline__ bool ngrid_in(const NGrid& g, int x, int y, int z) {
   return x >= 0 && y >= 0 && z >= 0 && x < g.X && y < g.Y && z < g.Z;
 }
@@ -53,201 +80,288 @@ struct ConvArgs {
   int acs, aco;
   int relu;
   int B;
+  VoxDiv od;  // of the output grid
 };
 
-template <int CINP, int NOUT, int MODE>
+// Voxel counts fit 32 bits throughout: 2^31 voxels would take more than 400 GB of activations.
+//
+// One wave: MT tiles of 16 consecutive voxels of the batch (over row ends: a 33-voxel row would
+// leave 15 of 48 rows of row tiles empty) x NTW of the NOUT/16 column tiles, the waves of a
+// workgroup sharing voxels where NTW < NOUT/16.  A lane's voxel and the 27 bits saying which of
+// its taps are inside the grid are found once; the loads of U steps of K (A rows from clamped
+// addresses, zeroed after) are all in flight before their products.  Latency bound the plain
+// form (a branch and an address division per step, one A tile per B load): us at 8 x 33^3
+// voxels, 16 -> 16 channels 64 -> 28, 48 -> 16 147 -> 69, 16 -> 48 149 -> 48.
+template <int CINP, int NOUT, int MODE, int MT, int NTW>
 __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
-  constexpr int NT = NOUT / 16;
-  constexpr int KP = ((27 * CINP + 31) / 32) * 32;
+  constexpr int NT = NOUT / 16, NS = NT / NTW;
+  constexpr int KP = ((27 * CINP + 31) / 32) * 32, KC = KP / 32, U = MT == 1 ? 4 : 2;
   const int lane = threadIdx.x & 63, g = lane >> 4, i16 = lane & 15;
-  const int tpr = (a.go.X + 15) >> 4;
-  const int64_t tile = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int64_t ntile = (int64_t)a.B * a.go.Z * a.go.Y * tpr;
-  if (tile >= ntile) return;  // uniform per wave
-  int64_t t = tile;
-  const int tx = (int)(t % tpr);
-  t /= tpr;
-  const int oy = (int)(t % a.go.Y);
-  t /= a.go.Y;
-  const int oz = (int)(t % a.go.Z);
-  const int b = (int)(t / a.go.Z);
-  const int ox = tx * 16 + i16;
-  const bool rowok = ox < a.go.X;
+  const uint32_t wid = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int n0 = (int)(wid % NS) * NTW;
+  const uint32_t Vo = (uint32_t)a.go.X * a.go.Y * a.go.Z, NV = Vo * a.B, v0 = wid / NS * (16 * MT);
+  if (v0 >= NV) return;  // uniform per wave
   const int64_t Vi = (int64_t)a.gi.X * a.gi.Y * a.gi.Z;
-  const uint16_t* xb = a.x + (int64_t)b * Vi * a.xcs + a.xco;
-  f32x4_t acc[NT];
+  const uint16_t* base[MT];
+  uint32_t okm[MT];
 #pragma unroll
-  for (int n = 0; n < NT; ++n) acc[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  for (int kc = 0; kc < KP; kc += 32) {
-    const int k0 = kc + 8 * g;
-    const int tap = k0 / CINP, ci = k0 % CINP;
-    uint4 av = make_uint4(0, 0, 0, 0);
-    if (tap < 27 && rowok) {
+  for (int m = 0; m < MT; ++m) {
+    const uint32_t v = v0 + 16 * m + i16, vc = v < NV ? v : NV - 1;
+    int ox, oy, oz;
+    const int b = vox_at(a.od, vc, ox, oy, oz);
+    // bit d of the axis: tap d - 1 reads inside the grid
+    const auto bits = [](int o, int n) {
+      uint32_t m3 = 0;
+#pragma unroll
+      for (int d = -1; d <= 1; ++d) {
+        int i = MODE == 0 ? o + d : (MODE == 1 ? 2 * o + d : o - d);
+        bool ok = true;
+        if (MODE == 3) {
+          ok = (i & 1) == 0;
+          i >>= 1;
+        }
+        if (ok && i >= 0 && i < n) m3 |= 1u << (d + 1);
+      }
+      return m3;
+    };
+    const uint32_t bx = bits(ox, a.gi.X), by = bits(oy, a.gi.Y), bz = bits(oz, a.gi.Z);
+    const uint32_t pl = ((by & 1) ? bx : 0u) | ((by & 2) ? bx << 3 : 0u) | ((by & 4) ? bx << 6 : 0u);
+    okm[m] = v < NV ? ((bz & 1) ? pl : 0u) | ((bz & 2) ? pl << 9 : 0u) | ((bz & 4) ? pl << 18 : 0u) : 0u;
+    const int ix = MODE == 1 ? 2 * ox : (MODE == 3 ? ox >> 1 : ox), iy = MODE == 1 ? 2 * oy : (MODE == 3 ? oy >> 1 : oy),
+              iz = MODE == 1 ? 2 * oz : (MODE == 3 ? oz >> 1 : oz);
+    base[m] = a.x + ((int64_t)b * Vi + ((int64_t)iz * a.gi.Y + iy) * a.gi.X + ix) * a.xcs + a.xco;
+  }
+  // stride-2 data gradients: most taps are odd for all of a wave's voxels; their steps are skipped
+  uint32_t any = 0;
+  if constexpr (MODE == 3) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m) any |= okm[m];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) any |= __shfl_xor(any, o, 64);
+    any = __builtin_amdgcn_readfirstlane(any);
+  }
+  f32x4_t acc[MT][NTW];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int n = 0; n < NTW; ++n) acc[m][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const uint16_t* wr = a.w + (int64_t)(n0 * 16 + i16) * KP;
+  for (int kc = 0; kc < KC; kc += U) {
+    if constexpr (MODE == 3) {
+      const int t0 = kc * 32 / CINP, t1 = min(26, ((kc + U) * 32 - 1) / CINP);
+      if (!((any >> t0) & ((2u << (t1 - t0)) - 1))) continue;
+    }
+    uint4 av[U][MT], bv[U][NTW];
+    uint32_t ok[U][MT];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k0 = 32 * (kc + u) + 8 * g, tap = k0 / CINP, ci = k0 % CINP;
       const int dx = tap % 3 - 1, dy = (tap / 3) % 3 - 1, dz = tap / 9 - 1;
-      int ix, iy, iz;
-      bool ok = true;
-      if (MODE == 0) {
-        ix = ox + dx; iy = oy + dy; iz = oz + dz;
-      } else if (MODE == 1) {
-        ix = 2 * ox + dx; iy = 2 * oy + dy; iz = 2 * oz + dz;
-      } else if (MODE == 2) {
-        ix = ox - dx; iy = oy - dy; iz = oz - dz;
-      } else {
-        const int sx = ox - dx, sy = oy - dy, sz = oz - dz;
-        ok = ((sx | sy | sz) & 1) == 0;
-        ix = sx >> 1; iy = sy >> 1; iz = sz >> 1;
-      }
-      if (ok && ngrid_in(a.gi, ix, iy, iz))
-        av = *(const uint4*)(xb + (((int64_t)iz * a.gi.Y + iy) * a.gi.X + ix) * a.xcs + ci);
-    }
-    const bf16x8_t A = __builtin_bit_cast(bf16x8_t, av);
+      const int vo = MODE == 3 ? (dx < 0) + a.gi.X * ((dy < 0) + a.gi.Y * (dz < 0)) : dx + a.gi.X * (dy + a.gi.Y * dz);
+      const int off = (MODE == 2 ? -vo : vo) * a.xcs + ci;
 #pragma unroll
-    for (int n = 0; n < NT; ++n) {
-      const uint4 bv = *(const uint4*)(a.w + (int64_t)(n * 16 + i16) * KP + k0);
-      acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, __builtin_bit_cast(bf16x8_t, bv), acc[n], 0, 0, 0);
+      for (int m = 0; m < MT; ++m) {
+        ok[u][m] = tap < 27 ? (okm[m] >> tap) & 1u : 0u;
+        av[u][m] = *(const uint4*)(base[m] + (ok[u][m] ? off : 0));
+      }
+#pragma unroll
+      for (int n = 0; n < NTW; ++n) bv[u][n] = *(const uint4*)(wr + (int64_t)n * 16 * KP + min(k0, KP - 32 + 8 * g));
     }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        const uint4 z = ok[u][m] ? av[u][m] : make_uint4(0, 0, 0, 0);
+#pragma unroll
+        for (int n = 0; n < NTW; ++n)
+          acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, z),
+                                                              __builtin_bit_cast(bf16x8_t, bv[u][n]), acc[m][n], 0, 0, 0);
+      }
   }
-  // lane holds D[row 4g + r][col i16]: voxel tx*16 + 4g + r, channel n*16 + i16
-  const int64_t Vo = (int64_t)a.go.X * a.go.Y * a.go.Z;
-  const int64_t vrow = (int64_t)b * Vo + ((int64_t)oz * a.go.Y + oy) * a.go.X;
+  // lane holds D[row 4g + r][col i16] of each tile: voxel 16 m + 4g + r, channel (n0 + n)*16 + i16
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int vx = tx * 16 + 4 * g + r;
-    if (vx >= a.go.X) continue;
-    const int64_t v = vrow + vx;
+  for (int m = 0; m < MT; ++m)
 #pragma unroll
-    for (int n = 0; n < NT; ++n) {
-      const int co = n * 16 + i16;
-      float val = acc[n][r];
-      if (a.bias) val += a.bias[co];
-      if (a.add) val += bf2f(a.add[v * a.acs + a.aco + co]);
-      if (a.relu) val = fmaxf(val, 0.f);
-      if (a.mask && !(bf2f(a.mask[v * a.mcs + a.mco + co]) > 0.f)) val = 0.f;
-      if (a.y32) {
-        if (co < a.nstore) a.y32[v * a.nstore + co] = val;
-      } else {
-        a.y[v * a.ycs + a.yco + co] = f2bf(val);
-      }
-    }
-  }
-}
-
-// weight gradient partials part[grp][tap][ci][co] (ci < CI16) over voxel tiles grp, grp+G, ...
-// x: forward input (stride xcs, offset xco) on grid gi; dy: gradient of the (pre-activation)
-// forward output, contiguous with NOUT channels, on grid go.
-template <int CINP, int NOUT, int STRIDE>
-__global__ __launch_bounds__(256) void k_conv_wgrad(const uint16_t* __restrict__ x, int xcs, int xco, NGrid gi,
-                                                    const uint16_t* __restrict__ dy, NGrid go, int B,
-                                                    float* __restrict__ part) {
-  constexpr int CI16 = ((CINP + 15) / 16) * 16;
-  constexpr int MT = CI16 / 16, NT = NOUT / 16, NTILE = MT * NT, PER = (NTILE + 3) / 4;
-  constexpr int LD = 64 + 8;  // row pitch (elements): 144 bytes, 16-byte aligned rows
-  __shared__ __attribute__((aligned(16))) uint16_t sx[CI16 * LD];
-  __shared__ __attribute__((aligned(16))) uint16_t sd[NOUT * LD];
-  const int tap = blockIdx.x, grp = blockIdx.y, G = gridDim.y;
-  const int dx = tap % 3 - 1, dy_ = (tap / 3) % 3 - 1, dz = tap / 9 - 1;
-  const int lane = threadIdx.x & 63, g = lane >> 4, i16 = lane & 15, wv = threadIdx.x >> 6;
-  const int64_t Vo = (int64_t)go.X * go.Y * go.Z, Vi = (int64_t)gi.X * gi.Y * gi.Z;
-  const int64_t NV = (int64_t)B * Vo, ntl = (NV + 63) / 64;
-  for (int q = threadIdx.x; q < CI16 * LD; q += 256) sx[q] = 0;
-  f32x4_t acc[PER];
+    for (int r = 0; r < 4; ++r) {
+      const uint32_t v32 = v0 + 16 * m + 4 * g + r;
+      if (v32 >= NV) continue;
+      const int64_t v = v32;
 #pragma unroll
-  for (int p = 0; p < PER; ++p) acc[p] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  __syncthreads();
-  for (int64_t tl = grp; tl < ntl; tl += G) {
-    const int64_t v0 = tl * 64;
-    for (int q = threadIdx.x; q < 64 * (NOUT / 8); q += 256) {
-      const int vv = q / (NOUT / 8), c8 = (q % (NOUT / 8)) * 8;
-      uint4 val = make_uint4(0, 0, 0, 0);
-      if (v0 + vv < NV) val = *(const uint4*)(dy + (v0 + vv) * NOUT + c8);
-      const uint16_t* h = (const uint16_t*)&val;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) sd[(c8 + j) * LD + vv] = h[j];
-    }
-    for (int q = threadIdx.x; q < 64 * (CINP / 8); q += 256) {
-      const int vv = q / (CINP / 8), c8 = (q % (CINP / 8)) * 8;
-      uint4 val = make_uint4(0, 0, 0, 0);
-      const int64_t v = v0 + vv;
-      if (v < NV) {
-        const int b = (int)(v / Vo);
-        int64_t r = v - (int64_t)b * Vo;
-        const int ox = (int)(r % go.X);
-        r /= go.X;
-        const int oy = (int)(r % go.Y), oz = (int)(r / go.Y);
-        const int ix = STRIDE * ox + dx, iy = STRIDE * oy + dy_, iz = STRIDE * oz + dz;
-        if (ngrid_in(gi, ix, iy, iz))
-          val = *(const uint4*)(x + ((int64_t)b * Vi + ((int64_t)iz * gi.Y + iy) * gi.X + ix) * xcs + xco + c8);
-      }
-      const uint16_t* h = (const uint16_t*)&val;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) sx[(c8 + j) * LD + vv] = h[j];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int p = 0; p < PER; ++p) {
-      const int tid = wv + 4 * p;
-      if (tid < NTILE) {
-        const int mt = tid / NT, nt = tid % NT;
-#pragma unroll
-        for (int ks = 0; ks < 64; ks += 32) {
-          const uint4 av = *(const uint4*)(sx + (mt * 16 + i16) * LD + ks + 8 * g);
-          const uint4 bv = *(const uint4*)(sd + (nt * 16 + i16) * LD + ks + 8 * g);
-          acc[p] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av),
-                                                           __builtin_bit_cast(bf16x8_t, bv), acc[p], 0, 0, 0);
+      for (int n = 0; n < NTW; ++n) {
+        const int co = (n0 + n) * 16 + i16;
+        float val = acc[m][n][r];
+        if (a.bias && co < a.nstore) val += a.bias[co];
+        if (a.add) val += bf2f(a.add[v * a.acs + a.aco + co]);
+        if (a.relu) val = fmaxf(val, 0.f);
+        if (a.mask && !(bf2f(a.mask[v * a.mcs + a.mco + co]) > 0.f)) val = 0.f;
+        if (a.y32) {
+          if (co < a.nstore) a.y32[v * a.nstore + co] = val;
+        } else {
+          a.y[v * a.ycs + a.yco + co] = f2bf(val);
         }
       }
     }
-    __syncthreads();
-  }
+}
+
+// weight gradient partials part[grp][tap][ci][co] (ci < CI16), the sum over the voxel tiles of
+// block (tap, grp); x: forward input (stride xcs, offset xco) on grid gi; dy: gradient of the
+// (pre-activation) forward output, contiguous with NOUT channels, on grid go.
+// Each wave takes tiles of 64 voxels of its own: it transposes them into its part of LDS, two
+// voxels per 32-bit write, forms all channel tiles and needs no workgroup barrier before the
+// waves' sums are added at the end; the next tile's loads are in flight during the products.
+// (One tile per workgroup left three of four waves idle at 16 x 16 channels and met two
+// barriers a tile: us at 8 x 33^3 voxels 16 x 16 97 -> 44, 48 x 16 236 -> 92, 96 x 32 at
+// 8 x 17^3 101 -> 41; the runtime divisions of a voxel's coordinates alone were 8 of them.)
+template <int CINP, int NOUT, int STRIDE>
+__global__ __launch_bounds__(256) void k_conv_wgrad(const uint16_t* __restrict__ x, int xcs, int xco, NGrid gi,
+                                                    const uint16_t* __restrict__ dy, NGrid go, VoxDiv od, int B,
+                                                    float* __restrict__ part) {
+  constexpr int CI16 = ((CINP + 15) / 16) * 16;
+  constexpr int MT = CI16 / 16, NT = NOUT / 16;
+  constexpr int LD = 64 + 8;  // row pitch (elements): 144 bytes, 16-byte aligned rows
+  constexpr int GX = CINP / 8, GD = NOUT / 8, JX = (GX + 1) / 2, JD = GD / 2;
+  __shared__ __attribute__((aligned(16))) uint16_t slab[4][(CI16 + NOUT) * LD];
+  static_assert(CI16 * NOUT * 4 <= sizeof(slab[0]), "the sums take the tiles' place");
+  const int tap = blockIdx.x, grp = blockIdx.y, G = gridDim.y;
+  const int dx = tap % 3 - 1, dy_ = (tap / 3) % 3 - 1, dz = tap / 9 - 1;
+  const int lane = threadIdx.x & 63, g = lane >> 4, i16 = lane & 15, wv = threadIdx.x >> 6;
+  uint16_t *sx = slab[wv], *sd = sx + CI16 * LD;
+  const uint32_t Vo = (uint32_t)go.X * go.Y * go.Z, NV = Vo * B, ntl = (NV + 63) / 64;
+  const int64_t Vi = (int64_t)gi.X * gi.Y * gi.Z;
+  if constexpr (CI16 != CINP)
+    for (int q = lane; q < CI16 * LD; q += 64) sx[q] = 0;
+  f32x4_t acc[MT][NT];
 #pragma unroll
-  for (int p = 0; p < PER; ++p) {
-    const int tid = wv + 4 * p;
-    if (tid < NTILE) {
-      const int mt = tid / NT, nt = tid % NT;
+  for (int m = 0; m < MT; ++m)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int ci = mt * 16 + 4 * g + r, co = nt * 16 + i16;
-        part[(((int64_t)grp * 27 + tap) * CI16 + ci) * NOUT + co] = acc[p][r];
-      }
+    for (int n = 0; n < NT; ++n) acc[m][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  // lane: voxels 2 (lane % 32) and the next, channel groups lane / 32 + 2 j
+  const int pr = lane & 31, hf = lane >> 5;
+  uint4 rx[JX][2], rd[JD][2];
+  bool kx[2], kd[2];
+  const auto fetch = [&](uint32_t tl) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const uint32_t v = tl * 64 + 2 * pr + e;
+      int ox, oy, oz;
+      const int b = vox_at(od, v, ox, oy, oz);
+      const int ix = STRIDE * ox + dx, iy = STRIDE * oy + dy_, iz = STRIDE * oz + dz;
+      kd[e] = v < NV;
+      kx[e] = kd[e] && ngrid_in(gi, ix, iy, iz);
+      const uint16_t* px = x + (kx[e] ? (int64_t)b * Vi + ((int64_t)iz * gi.Y + iy) * gi.X + ix : 0) * xcs + xco;
+      const uint16_t* pd = dy + (int64_t)(kd[e] ? v : 0) * NOUT;
+#pragma unroll
+      for (int j = 0; j < JX; ++j) rx[j][e] = *(const uint4*)(px + 8 * min(hf + 2 * j, GX - 1));
+#pragma unroll
+      for (int j = 0; j < JD; ++j) rd[j][e] = *(const uint4*)(pd + 8 * (hf + 2 * j));
     }
+  };
+  // channel k of the two voxels, side by side, in row (8 c + k) of a tile
+  const auto put = [&](uint16_t* t, int c, uint4 a, uint4 b) {
+    const uint32_t va[4] = {a.x, a.y, a.z, a.w}, vb[4] = {b.x, b.y, b.z, b.w};
+    uint32_t* w = (uint32_t*)t + (8 * c) * (LD / 2) + pr;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      w[(2 * k) * (LD / 2)] = (va[k] & 0xffffu) | (vb[k] << 16);
+      w[(2 * k + 1) * (LD / 2)] = (va[k] >> 16) | (vb[k] & 0xffff0000u);
+    }
+  };
+  const uint4 zero = make_uint4(0, 0, 0, 0);
+  uint32_t tl = 4 * grp + wv;
+  if (tl < ntl) fetch(tl);
+  for (; tl < ntl; tl += 4 * G) {
+#pragma unroll
+    for (int j = 0; j < JX; ++j)
+      if (hf + 2 * j < GX) put(sx, hf + 2 * j, kx[0] ? rx[j][0] : zero, kx[1] ? rx[j][1] : zero);
+#pragma unroll
+    for (int j = 0; j < JD; ++j) put(sd, hf + 2 * j, kd[0] ? rd[j][0] : zero, kd[1] ? rd[j][1] : zero);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (tl + 4 * G < ntl) fetch(tl + 4 * G);
+#pragma unroll
+    for (int ks = 0; ks < 64; ks += 32) {
+      bf16x8_t A[MT], D[NT];
+#pragma unroll
+      for (int m = 0; m < MT; ++m) A[m] = *(const bf16x8_t*)(sx + (m * 16 + i16) * LD + ks + 8 * g);
+#pragma unroll
+      for (int n = 0; n < NT; ++n) D[n] = *(const bf16x8_t*)(sd + (n * 16 + i16) * LD + ks + 8 * g);
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[m], D[n], acc[m][n], 0, 0, 0);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   }
+  float* sum = (float*)slab[wv];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sum[(m * 16 + 4 * g + r) * NOUT + n * 16 + i16] = acc[m][n][r];
+  __syncthreads();
+  for (int q = threadIdx.x; q < CI16 * NOUT; q += 256)
+    part[((int64_t)grp * 27 + tap) * CI16 * NOUT + q] =
+        (((const float*)slab[0])[q] + ((const float*)slab[1])[q]) + (((const float*)slab[2])[q] + ((const float*)slab[3])[q]);
 }
 
-// grad[woff + (tap*cin + ci)*cout + co] = sum_grp part[grp][tap][ci][co]  (fixed order)
-__global__ void k_wgrad_fold(const float* __restrict__ part, int G, int ci16, int nout, int cin, int cout,
-                             float* __restrict__ grad) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t n = 27LL * cin * cout;
-  if (i >= n) return;
-  const int co = (int)(i % cout), ci = (int)((i / cout) % cin), tap = (int)(i / ((int64_t)cout * cin));
-  float s = 0.f;
-  for (int gq = 0; gq < G; ++gq) s += part[(((int64_t)gq * 27 + tap) * ci16 + ci) * nout + co];
-  grad[i] = s;
-}
-
-// bias gradient: part[grp][co] = sum over voxels grp, grp+G, ... of dy[v][co]
+// Bias gradient partials: part[grp][co] = sum of dy[v][co] over the voxels of block grp, eight
+// channels per load (64 blocks of 2-byte loads took 37 us at 8 x 33^3 x 16, these 6).
 __global__ __launch_bounds__(256) void k_bias_grad(const uint16_t* __restrict__ dy, int64_t NV, int nout,
                                                    float* __restrict__ part) {
-  __shared__ float sh[256];
-  const int per = 256 / nout, co = threadIdx.x % nout, sub = threadIdx.x / nout;
-  float s = 0.f;
-  if (sub < per)
-    for (int64_t v = (int64_t)blockIdx.x * per + sub; v < NV; v += (int64_t)gridDim.x * per)
-      s += bf2f(dy[v * nout + co]);
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  if (threadIdx.x < nout) {
-    float t = 0.f;
-    for (int j = 0; j < per; ++j) t += sh[j * nout + threadIdx.x];
-    part[(int64_t)blockIdx.x * nout + threadIdx.x] = t;
+  __shared__ float sh[4][64];
+  const int c8n = nout / 8, per = 256 / c8n, c8 = threadIdx.x % c8n, lane = threadIdx.x & 63;  // c8n: 2, 4 or 8
+  float s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll 4
+  for (int64_t v = (int64_t)blockIdx.x * per + threadIdx.x / c8n; v < NV; v += (int64_t)gridDim.x * per) {
+    const uint4 val = *(const uint4*)(dy + v * nout + 8 * c8);
+    const uint16_t* h = (const uint16_t*)&val;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) s[k] += bf2f(h[k]);
   }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    for (int o = 32; o >= c8n; o >>= 1) s[k] += __shfl_xor(s[k], o, 64);
+    if (lane < c8n) sh[threadIdx.x >> 6][8 * lane + k] = s[k];
+  }
+  __syncthreads();
+  if (threadIdx.x < nout)
+    part[(int64_t)blockIdx.x * nout + threadIdx.x] =
+        (sh[0][threadIdx.x] + sh[1][threadIdx.x]) + (sh[2][threadIdx.x] + sh[3][threadIdx.x]);
 }
-__global__ void k_bias_fold(const float* __restrict__ part, int G, int nout, int cout, float* __restrict__ grad) {
-  const int co = threadIdx.x;
-  if (co >= cout) return;
+
+// folds a layer's partials in a fixed order: grad[(tap*cin + ci)*cout + co] from the GW weight
+// groups, and in the launch's last block gbias[co] from the GB bias groups (one launch where
+// there were two, their loads in flight together: 17 + 15 -> 7 us)
+__global__ __launch_bounds__(256) void k_grad_fold(const float* __restrict__ part, int GW, int ci16, int nout, int cin,
+                                                   int cout, float* __restrict__ grad, const float* __restrict__ bpart,
+                                                   int GB, float* __restrict__ gbias) {
+  if (blockIdx.x + 1 == gridDim.x) {
+    __shared__ float sh[256];
+    const int co = threadIdx.x % nout, per = 256 / nout;  // nout: 16, 32 or 64
+    float s = 0.f;
+#pragma unroll 8
+    for (int q = threadIdx.x / nout; q < GB; q += per) s += bpart[(int64_t)q * nout + co];
+    sh[threadIdx.x] = s;
+    __syncthreads();
+    if (threadIdx.x < cout) {
+      float t = 0.f;
+      for (int j = 0; j < per; ++j) t += sh[j * nout + threadIdx.x];
+      gbias[threadIdx.x] = t;
+    }
+    return;
+  }
+  // 64 weights per block, a quarter of the groups per wave
+  __shared__ float sw[4][64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t i = (int64_t)blockIdx.x * 64 + lane, n = 27LL * cin * cout, ic = i < n ? i : n - 1;
+  const int co = (int)(ic % cout), ci = (int)((ic / cout) % cin), tap = (int)(ic / ((int64_t)cout * cin));
   float s = 0.f;
-  for (int gq = 0; gq < G; ++gq) s += part[(int64_t)gq * nout + co];
-  grad[co] = s;
+#pragma unroll 16
+  for (int q = wv; q < GW; q += 4) s += part[(((int64_t)q * 27 + tap) * ci16 + ci) * nout + co];
+  sw[wv][lane] = s;
+  __syncthreads();
+  if (wv == 0 && i < n) grad[i] = (sw[0][lane] + sw[1][lane]) + (sw[2][lane] + sw[3][lane]);
 }
 
 // BF16 weight copies from the FP32 master W[tap][ci][co]:

@@ -85,7 +85,7 @@ struct tos_dataset {
 namespace {
 
 constexpr int kWgradGroups = 64;
-constexpr int kBiasGroups = 64;
+constexpr int kBiasGroups = 256;
 
 template <class T>
 T* nalloc(std::vector<void*>& list, hipStream_t s, size_t n) {
@@ -214,30 +214,38 @@ void unet_prep(tos_unet* N, hipStream_t st) {
 }
 
 // ---- convolution dispatch -------------------------------------------------------------
-#define TOS_CONV_CASE(CI, NO, MD)                                                  \
-  if (cinp == CI && nout == NO && mode == MD) {                                    \
-    hipLaunchKernelGGL((k_conv<CI, NO, MD>), dim3(blocks), dim3(256), 0, st, a);   \
-    return;                                                                        \
+// NTW column tiles per wave; four voxel tiles per wave where that leaves four waves per SIMD
+// (2^18 voxels), else one
+#define TOS_CONV_CASE(CI, NO, MD, NTW)                                                              \
+  if (cinp == CI && nout == NO && mode == MD) {                                                     \
+    constexpr int NS = NO / 16 / NTW;                                                               \
+    if (nv * NS >= kConvWide)                                                                       \
+      hipLaunchKernelGGL((k_conv<CI, NO, MD, 4, NTW>), dim3((unsigned)(((nv + 63) / 64 * NS + 3) / 4)), dim3(256), 0, \
+                         st, a);                                                                    \
+    else                                                                                            \
+      hipLaunchKernelGGL((k_conv<CI, NO, MD, 1, NTW>), dim3((unsigned)(((nv + 15) / 16 * NS + 3) / 4)), dim3(256), 0, \
+                         st, a);                                                                    \
+    return;                                                                                         \
   }
+constexpr int64_t kConvWide = 1 << 18;
 void conv_launch(int cinp, int nout, int mode, const tos::ConvArgs& a, hipStream_t st) {
-  const int64_t tiles = (int64_t)a.B * a.go.Z * a.go.Y * ((a.go.X + 15) / 16);
-  const unsigned blocks = (unsigned)((tiles + 3) / 4);
-  if (blocks == 0) return;
-  TOS_CONV_CASE(8, 16, 0)
-  TOS_CONV_CASE(16, 16, 0)
-  TOS_CONV_CASE(16, 32, 1)
-  TOS_CONV_CASE(32, 32, 0)
-  TOS_CONV_CASE(32, 64, 1)
-  TOS_CONV_CASE(64, 64, 0)
-  TOS_CONV_CASE(96, 32, 0)
-  TOS_CONV_CASE(48, 16, 0)
-  TOS_CONV_CASE(16, 16, 2)
-  TOS_CONV_CASE(16, 48, 2)
-  TOS_CONV_CASE(32, 32, 2)
-  TOS_CONV_CASE(32, 96, 2)
-  TOS_CONV_CASE(64, 64, 2)
-  TOS_CONV_CASE(64, 32, 3)
-  TOS_CONV_CASE(32, 16, 3)
+  const int64_t nv = (int64_t)a.B * a.go.Z * a.go.Y * a.go.X;
+  if (nv == 0) return;
+  TOS_CONV_CASE(8, 16, 0, 1)
+  TOS_CONV_CASE(16, 16, 0, 1)
+  TOS_CONV_CASE(16, 32, 1, 2)
+  TOS_CONV_CASE(32, 32, 0, 2)
+  TOS_CONV_CASE(32, 64, 1, 1)
+  TOS_CONV_CASE(64, 64, 0, 1)
+  TOS_CONV_CASE(96, 32, 0, 2)
+  TOS_CONV_CASE(48, 16, 0, 1)
+  TOS_CONV_CASE(16, 16, 2, 1)
+  TOS_CONV_CASE(16, 48, 2, 3)
+  TOS_CONV_CASE(32, 32, 2, 2)
+  TOS_CONV_CASE(32, 96, 2, 3)
+  TOS_CONV_CASE(64, 64, 2, 1)
+  TOS_CONV_CASE(64, 32, 3, 2)
+  TOS_CONV_CASE(32, 16, 3, 1)
   throw std::runtime_error("conv: unsupported shape " + std::to_string(cinp) + "x" + std::to_string(nout) +
                            " mode " + std::to_string(mode));
 }
@@ -246,7 +254,7 @@ void conv_launch(int cinp, int nout, int mode, const tos::ConvArgs& a, hipStream
 #define TOS_WGRAD_CASE(CI, NO, S)                                                                      \
   if (cinp == CI && nout == NO && stride == S) {                                                       \
     hipLaunchKernelGGL((k_conv_wgrad<CI, NO, S>), dim3(27, kWgradGroups), dim3(256), 0, st, x, xcs, xco, gi, dy, \
-                       go, B, part);                                                                   \
+                       go, tos::vox_div(go), B, part);                                                                   \
     return;                                                                                            \
   }
 void wgrad_launch(int cinp, int nout, int stride, const uint16_t* x, int xcs, int xco, tos::NGrid gi,
@@ -267,6 +275,7 @@ tos::ConvArgs conv_args(int B, const uint16_t* x, int xcs, int xco, tos::NGrid g
                         tos::NGrid go) {
   tos::ConvArgs a{};
   a.x = x; a.xcs = xcs; a.xco = xco; a.gi = gi; a.w = w; a.go = go; a.B = B;
+  a.od = tos::vox_div(go);
   return a;
 }
 
@@ -325,12 +334,10 @@ void layer_wgrad(tos_unet* N, int li, int B, const uint16_t* x, int xcs, int xco
   wgrad_launch(L.cinp, L.nout, L.stride, x, xcs, xco, gi, dy, go, B, N->wpart, st);
   const int ci16 = (L.cinp + 15) / 16 * 16;
   const int64_t nw = 27LL * L.cin * L.cout;
-  hipLaunchKernelGGL(k_wgrad_fold, dim3(nblk(nw)), dim3(256), 0, st, (const float*)N->wpart, kWgradGroups, ci16,
-                     L.nout, L.cin, L.cout, N->grad + L.woff);
   hipLaunchKernelGGL(k_bias_grad, dim3(kBiasGroups), dim3(256), 0, st, dy, (int64_t)B * tos::ngrid_v(go), L.nout,
                      N->bpart);
-  hipLaunchKernelGGL(k_bias_fold, dim3(1), dim3(64), 0, st, (const float*)N->bpart, kBiasGroups, L.nout, L.cout,
-                     N->grad + L.boff);
+  hipLaunchKernelGGL(k_grad_fold, dim3(nblk(nw, 64) + 1), dim3(256), 0, st, (const float*)N->wpart, kWgradGroups, ci16,
+                     L.nout, L.cin, L.cout, N->grad + L.woff, (const float*)N->bpart, kBiasGroups, N->grad + L.boff);
 }
 
 // gradient of the loss w.r.t. all parameters, from A->gy (the loss kernel's output)
