@@ -4,27 +4,44 @@
 // The reference evaluates every vector expression of the primal-dual Newton iteration as
 // its own kernel (dozens per step) and solves the (m+1)x(m+1) reduced system on the host.
 // Here each n-length sweep of a Newton step is one fused grid-stride kernel over the whole
-// GPU that also produces the step's reductions as fixed-order per-block partials; one
-// block folds them and the host reads the few scalars that steer the iteration (the
-// small system, the step bound, the KKT line search), exactly in the reference's order.
+// GPU that also produces the step's reductions as fixed-order per-block partials, which one
+// wave per column folds; the host reads the few scalars that steer the iteration.  It waits
+// twice per Newton step: for the sums of the reduced system and the KKT residual at the
+// current point (k_mma_point), and for the residuals of the line search (k_mma_trials: the
+// step bound is taken on the device and the first kTrials halvings are tried together).  With
+// a wait per sweep and trial, 5.3 a step, the 40 steps of the first update of 9537 coefficients
+// spent more time between kernels than in them; a TO iteration at 128x64x64 went from 12.5 to
+// 10.0 ms with two.
 #include "tos_internal.hpp"
 
 namespace tos {
 
 constexpr int MMAX = 4;       // constraints supported
-constexpr int MMA_CNT = 24;   // widest reduction (m + m*m + m for m = 4)
+constexpr int kTrials = 4;    // line-search steps tried together
+// columns of the reductions: sums first, then the maxima
+constexpr int kkt_cols(int m) { return 6 + m; }                   // 3 sums, m proxies, 3 maxima
+constexpr int point_cols(int m) { return m * m + m + kkt_cols(m); }
+constexpr int MMA_CNT = 4 + kTrials * kkt_cols(MMAX);             // widest: step bound and trials
+static_assert(MMA_CNT >= point_cols(MMAX), "reduction buffer");
 
 struct MmaVecs {
   int n, m;
   double *x, *xmin, *xmax, *L, *U, *alpha, *beta, *lastdx, *xi, *eta;
   double *p, *q;  // (m+1) x n
-  double *plam, *qlam, *curx, *Dx, *G, *dlx, *dx, *dxi, *deta, *tx, *txi, *teta;
+  double *curx, *Dx, *G, *dlx, *dx, *dxi, *deta;
 };
 
 struct MmaSmall {  // scalars passed by value
   double lam[MMAX], dlam[MMAX];
   double eps, step, move;
 };
+
+// lambda at a trial step, rounded as the host rounds it (product, then sum)
+__device__ __forceinline__ double mma_lam_at(double lam, double dlam, double step) {
+#pragma clang fp contract(off)
+  const double d = dlam * step;
+  return lam + d;
+}
 
 __device__ __forceinline__ int64_t mtid() { return (int64_t)blockIdx.x * blockDim.x + threadIdx.x; }
 __device__ __forceinline__ int64_t mstride() { return (int64_t)gridDim.x * blockDim.x; }
@@ -80,49 +97,77 @@ __global__ __launch_bounds__(256) void k_mma_pq(MmaVecs V, const double* __restr
   block_partials<MMAX>(v, mx, partial);
 }
 
-// Dx, delta_x and G at the current point; sums for the reduced system (mma_t.cu:358-395,
-// solveLinearSystem :228-328): proxies g_i, A11 = G Dx^-1 G^T, b1 part G (delta_x / Dx).
-__global__ __launch_bounds__(256) void k_mma_passA(MmaVecs V, MmaSmall S, double* partial) {
-  const int n = V.n, m = V.m;
-  constexpr int CA = MMAX + MMAX * MMAX + MMAX;
-  double v[CA];
-  bool mx[CA];
+// The current point (moved by S.step along the Newton direction first, unless 0) with the
+// multipliers S.lam: Dx, delta_x and G there, the sums of the reduced system (mma_t.cu:358-395,
+// solveLinearSystem :228-328), A11 = G Dx^-1 G^T in columns 0 .. m*m - 1 and b1's part
+// G (delta_x / Dx) in the next m, and the n-length parts of the KKT residual (kkt_err
+// mma_t.cu:574-678) in the rest: three sums of squares, the m proxies g_i, three maxima.
+template <int M>
+__global__ __launch_bounds__(256) void k_mma_point(MmaVecs V, MmaSmall S, double* partial) {
+  const int n = V.n;
+  constexpr int C = point_cols(M), K = M * M + M;
+  double v[C];
+  bool mx[C];
 #pragma unroll
-  for (int i = 0; i < CA; ++i) { v[i] = 0; mx[i] = false; }
+  for (int i = 0; i < C; ++i) { v[i] = 0; mx[i] = i >= C - 3; }
   for (int64_t j = mtid(); j < n; j += mstride()) {
-    const double xj = V.x[j], ux = V.U[j] - xj, xl = xj - V.L[j];
-    const double xa = xj - V.alpha[j], bx = V.beta[j] - xj;
-    const double psi = 2 * V.plam[j] / (ux * ux * ux) + 2 * V.qlam[j] / (xl * xl * xl);
-    const double Dx = psi + V.xi[j] / xa + V.eta[j] / bx;
-    const double phi = V.plam[j] / (ux * ux) - V.qlam[j] / (xl * xl);
+    double X = V.x[j], XI = V.xi[j], ETA = V.eta[j];
+    if (S.step != 0) {
+      X = fma(V.dx[j], S.step, X);
+      XI = fma(V.dxi[j], S.step, XI);
+      ETA = fma(V.deta[j], S.step, ETA);
+      V.x[j] = X; V.xi[j] = XI; V.eta[j] = ETA;
+    }
+    double pl = V.p[j], ql = V.q[j], pi[M], qi[M];
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+      pi[i] = V.p[(int64_t)(i + 1) * n + j];
+      qi[i] = V.q[(int64_t)(i + 1) * n + j];
+      pl += S.lam[i] * pi[i];
+      ql += S.lam[i] * qi[i];
+    }
+    const double ux = V.U[j] - X, xl = X - V.L[j];
+    const double xa = X - V.alpha[j], bx = V.beta[j] - X;
+    const double psi = 2 * pl / (ux * ux * ux) + 2 * ql / (xl * xl * xl);
+    const double Dx = psi + XI / xa + ETA / bx;
+    const double phi = pl / (ux * ux) - ql / (xl * xl);
     const double dlx = -(S.eps / xa - S.eps / bx - phi);
     V.Dx[j] = Dx;
     V.dlx[j] = dlx;
-    double Gi[MMAX];
-    for (int i = 0; i < m; ++i) {
-      const double pi = V.p[(int64_t)(i + 1) * n + j], qi = V.q[(int64_t)(i + 1) * n + j];
-      Gi[i] = pi / (ux * ux) - qi / (xl * xl);
+    double Gi[M];
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+      Gi[i] = pi[i] / (ux * ux) - qi[i] / (xl * xl);
       V.G[(int64_t)i * n + j] = Gi[i];
-      v[i] += pi / ux + qi / xl;
+      v[K + 3 + i] += pi[i] / ux + qi[i] / xl;
     }
-    for (int i = 0; i < m; ++i) {
-      for (int k = 0; k < m; ++k) v[MMAX + i * MMAX + k] += Gi[i] * (Gi[k] / Dx);
-      v[MMAX + MMAX * MMAX + i] += Gi[i] * (dlx / Dx);
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+#pragma unroll
+      for (int k = 0; k < M; ++k) v[i * M + k] += Gi[i] * (Gi[k] / Dx);
+      v[M * M + i] += Gi[i] * (dlx / Dx);
     }
+    const double rx = phi - XI + ETA, r1 = XI * xa - S.eps, r2 = ETA * bx - S.eps;
+    v[K] += rx * rx; v[K + 1] += r1 * r1; v[K + 2] += r2 * r2;
+    v[C - 3] = fmax(v[C - 3], fabs(rx));
+    v[C - 2] = fmax(v[C - 2], fabs(r1));
+    v[C - 1] = fmax(v[C - 1], fabs(r2));
   }
-  block_partials<CA>(v, mx, partial);
+  block_partials<C>(v, mx, partial);
 }
 
 // Newton direction in x, xi, eta and the fraction-to-boundary bounds (mma_t.cu:302-317,
 // :396-402)
-__global__ __launch_bounds__(256) void k_mma_passB(MmaVecs V, MmaSmall S, double* partial) {
-  const int n = V.n, m = V.m;
+template <int M>
+__global__ __launch_bounds__(256) void k_mma_direction(MmaVecs V, MmaSmall S, double* partial) {
+  const int n = V.n;
   double t[3] = {-1e300, -1e300, -1e300};
   const bool mx[3] = {true, true, true};
   const double cf = 1.0 / 0.99;
   for (int64_t j = mtid(); j < n; j += mstride()) {
     double dxv = -V.dlx[j] / V.Dx[j];
-    for (int i = 0; i < m; ++i) dxv -= S.dlam[i] * V.G[(int64_t)i * n + j] / V.Dx[j];
+#pragma unroll
+    for (int i = 0; i < M; ++i) dxv -= S.dlam[i] * V.G[(int64_t)i * n + j] / V.Dx[j];
     const double xa = V.x[j] - V.alpha[j], bx = V.beta[j] - V.x[j];
     const double dxi = S.eps / xa - dxv / xa * V.xi[j] - V.xi[j];
     const double deta = S.eps / bx + V.eta[j] / bx * dxv - V.eta[j];
@@ -136,66 +181,83 @@ __global__ __launch_bounds__(256) void k_mma_passB(MmaVecs V, MmaSmall S, double
   block_partials<3>(t, mx, partial);
 }
 
-// plam/qlam for lambda, then the n-length parts of the KKT residual (kkt_err
-// mma_t.cu:574-678) at the current point (TRIAL = false) or at the trial point
-// x + step dx (TRIAL = true, written to tx/txi/teta).
-template <bool TRIAL>
-__global__ __launch_bounds__(256) void k_mma_kkt(MmaVecs V, MmaSmall S, double* partial) {
-  const int n = V.n, m = V.m;
-  constexpr int CK = 3 + MMAX + 3;
-  double v[CK];
-  bool mx[CK];
+// folds the three bounds of k_mma_direction into out[0 .. 2] and the step into out[3]:
+// 1 / max(x bounds, max(xi and eta bound, the scalars' bound sb))
+__global__ __launch_bounds__(192) void k_mma_step(const double* __restrict__ partial, int nb, double sb,
+                                                  double* __restrict__ out) {
+  __shared__ double sh[3];
+  const int c = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  double s = -HUGE_VAL;
+  for (int b = lane; b < nb; b += 64) s = fmax(s, partial[(int64_t)c * nb + b]);
 #pragma unroll
-  for (int i = 0; i < CK; ++i) { v[i] = 0; mx[i] = i >= 3 + MMAX; }
-  for (int64_t j = mtid(); j < n; j += mstride()) {
-    double X = V.x[j], XI = V.xi[j], ETA = V.eta[j];
-    if (TRIAL) {
-      X = X + V.dx[j] * S.step;
-      XI = XI + V.dxi[j] * S.step;
-      ETA = ETA + V.deta[j] * S.step;
-      V.tx[j] = X; V.txi[j] = XI; V.teta[j] = ETA;
-    }
-    double pl = V.p[j], ql = V.q[j];
-    for (int i = 0; i < m; ++i) {
-      pl += S.lam[i] * V.p[(int64_t)(i + 1) * n + j];
-      ql += S.lam[i] * V.q[(int64_t)(i + 1) * n + j];
-    }
-    V.plam[j] = pl;
-    V.qlam[j] = ql;
-    const double ux = V.U[j] - X, xl = X - V.L[j];
-    const double rx = pl / (ux * ux) - ql / (xl * xl) - XI + ETA;
-    const double r1 = XI * (X - V.alpha[j]) - S.eps;
-    const double r2 = ETA * (V.beta[j] - X) - S.eps;
-    v[0] += rx * rx; v[1] += r1 * r1; v[2] += r2 * r2;
-    for (int i = 0; i < m; ++i) v[3 + i] += V.p[(int64_t)(i + 1) * n + j] / ux + V.q[(int64_t)(i + 1) * n + j] / xl;
-    v[3 + MMAX] = fmax(v[3 + MMAX], fabs(rx));
-    v[4 + MMAX] = fmax(v[4 + MMAX], fabs(r1));
-    v[5 + MMAX] = fmax(v[5 + MMAX], fabs(r2));
-  }
-  block_partials<CK>(v, mx, partial);
+  for (int o = 32; o > 0; o >>= 1) s = fmax(s, __shfl_xor(s, o, 64));
+  if (lane == 0) sh[c] = out[c] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) out[3] = 1.0 / fmax(fmax(sh[0], sh[1]), fmax(sh[2], sb));
 }
 
-// plam/qlam only (after the reset, with lambda = 1)
-__global__ __launch_bounds__(256) void k_mma_plam(MmaVecs V, MmaSmall S) {
-  const int n = V.n, m = V.m;
-  for (int64_t j = mtid(); j < n; j += mstride()) {
-    double pl = V.p[j], ql = V.q[j];
-    for (int i = 0; i < m; ++i) {
-      pl += S.lam[i] * V.p[(int64_t)(i + 1) * n + j];
-      ql += S.lam[i] * V.q[(int64_t)(i + 1) * n + j];
-    }
-    V.plam[j] = pl;
-    V.qlam[j] = ql;
+// n-length parts of the KKT residual at x + t dx for the steps t = scale * step[0] / 2^k,
+// k < kTrials: columns k * kkt_cols(M) + (three sums of squares, proxies, three maxima)
+template <int M>
+__global__ __launch_bounds__(256) void k_mma_trials(MmaVecs V, MmaSmall S, const double* __restrict__ step,
+                                                    double scale, double* partial) {
+  const int n = V.n;
+  constexpr int CK = kkt_cols(M), C = kTrials * CK;
+  double t[kTrials], lam[kTrials][M];
+  t[0] = scale * step[0];
+#pragma unroll
+  for (int k = 0; k < kTrials; ++k) {
+    if (k > 0) t[k] = t[k - 1] / 2;
+#pragma unroll
+    for (int i = 0; i < M; ++i) lam[k][i] = mma_lam_at(S.lam[i], S.dlam[i], t[k]);
   }
+  double v[C];
+  bool mx[C];
+#pragma unroll
+  for (int i = 0; i < C; ++i) { v[i] = 0; mx[i] = i % CK >= CK - 3; }
+  for (int64_t j = mtid(); j < n; j += mstride()) {
+    const double x0 = V.x[j], xi0 = V.xi[j], eta0 = V.eta[j], dx = V.dx[j], dxi = V.dxi[j], deta = V.deta[j];
+    const double U = V.U[j], L = V.L[j], al = V.alpha[j], be = V.beta[j], p0 = V.p[j], q0 = V.q[j];
+    double pi[M], qi[M];
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+      pi[i] = V.p[(int64_t)(i + 1) * n + j];
+      qi[i] = V.q[(int64_t)(i + 1) * n + j];
+    }
+#pragma unroll
+    for (int k = 0; k < kTrials; ++k) {
+      const double X = fma(dx, t[k], x0), XI = fma(dxi, t[k], xi0), ETA = fma(deta, t[k], eta0);
+      double pl = p0, ql = q0;
+#pragma unroll
+      for (int i = 0; i < M; ++i) {
+        pl += lam[k][i] * pi[i];
+        ql += lam[k][i] * qi[i];
+      }
+      const double ux = U - X, xl = X - L;
+      const double rx = pl / (ux * ux) - ql / (xl * xl) - XI + ETA;
+      const double r1 = XI * (X - al) - S.eps, r2 = ETA * (be - X) - S.eps;
+      double* w = v + k * CK;
+      w[0] += rx * rx; w[1] += r1 * r1; w[2] += r2 * r2;
+#pragma unroll
+      for (int i = 0; i < M; ++i) w[3 + i] += pi[i] / ux + qi[i] / xl;
+      w[CK - 3] = fmax(w[CK - 3], fabs(rx));
+      w[CK - 2] = fmax(w[CK - 2], fabs(r1));
+      w[CK - 1] = fmax(w[CK - 1], fabs(r2));
+    }
+  }
+  block_partials<C>(v, mx, partial);
 }
 
-// asymptotes and move limits for the next iteration (adjust_asym mma_t.cu:164-226)
+// asymptotes and move limits for the next iteration (adjust_asym mma_t.cu:164-226), after the
+// last accepted Newton step S.step
 __global__ __launch_bounds__(256) void k_mma_asym(MmaVecs V, MmaSmall S, double* partial) {
   const int n = V.n;
   double v[1] = {0};
   const bool mx[1] = {false};
   for (int64_t j = mtid(); j < n; j += mstride()) {
-    const double xv = V.x[j], d1 = xv - V.curx[j], d2 = V.lastdx[j];
+    const double xv = S.step != 0 ? fma(V.dx[j], S.step, V.x[j]) : V.x[j];
+    V.x[j] = xv;
+    const double d1 = xv - V.curx[j], d2 = V.lastdx[j];
     double gam = 1;
     if (d1 * d2 > 0) gam = 1.2;
     if (d1 * d2 < 0) gam = 0.7;
@@ -222,11 +284,11 @@ __global__ __launch_bounds__(256) void k_mma_asym(MmaVecs V, MmaSmall S, double*
 
 // fold `cnt` columns of `nb` per-block partials in a fixed order: one 64-lane wave per
 // column (grid = cnt), lane-strided partial sums, then a fixed butterfly
-__global__ __launch_bounds__(64) void k_mma_fold(const double* __restrict__ partial, int nb, int cnt,
-                                                 unsigned maxmask, double* __restrict__ out) {
+// (every `period` columns the last `nmax` are maxima)
+__global__ __launch_bounds__(64) void k_mma_fold(const double* __restrict__ partial, int nb, int period, int nmax,
+                                                 double* __restrict__ out) {
   const int c = blockIdx.x;
-  if (c >= cnt) return;
-  const bool mx = (maxmask >> c) & 1u;
+  const bool mx = c % period >= period - nmax;
   const int lane = threadIdx.x;
   const double* col = partial + (int64_t)c * nb;
   double s = lane < nb ? col[lane] : (mx ? -HUGE_VAL : 0.0);

@@ -2430,57 +2430,53 @@ T* malloc_mma(tos_mma* M, size_t n) {
   return (T*)raw_alloc(M->allocs, M->stream, n * sizeof(T));
 }
 
-// run a pass kernel, fold its `cnt` columns, read them to M->h_red
+// run a pass kernel, fold its `cnt` columns (of every `period` the last `nmax` are maxima), read
+// them to M->h_red
 template <class K, class... A>
-const double* mma_pass(tos_mma* M, hipStream_t st, K kernel, int cnt, unsigned maxmask, A... args) {
+const double* mma_pass(tos_mma* M, hipStream_t st, K kernel, int cnt, int period, int nmax, A... args) {
   hipLaunchKernelGGL(kernel, dim3(M->nb), dim3(256), 0, st, args...);
-  hipLaunchKernelGGL(k_mma_fold, dim3(cnt), dim3(64), 0, st, (const double*)M->partial, M->nb, cnt, maxmask, M->red);
+  hipLaunchKernelGGL(k_mma_fold, dim3(cnt), dim3(64), 0, st, (const double*)M->partial, M->nb, period, nmax, M->red);
   LAUNCH_CHECK();
   download(st, M->h_red, M->red, cnt * sizeof(double));
   return M->h_red;
 }
 
-// KKT residual (2-norm, inf-norm) from the folded n-length parts and the scalars
+// KKT residual (2-norm, inf-norm) from the folded n-length parts v (kkt_cols) and the scalars
 // (kkt_err mma_t.cu:574-678, same order of accumulation)
 std::pair<double, double> mma_kkt_host(const tos_mma* M, const double* v, const double* y, const double* lam,
                                        const double* mu, const double* s, double z, double zeta, double damp) {
   const int m = M->V.m;
-  double sum = v[0], mx = std::max(-10.0, v[3 + MMAX]);
+  double sum = v[0], mx = std::max(-10.0, v[3 + m]);
   auto acc = [&](double r) { sum += r * r; mx = std::max(mx, std::fabs(r)); };
   for (int i = 0; i < m; ++i) acc(M->c[i] + M->d[i] * y[i] - lam[i] - mu[i]);
   double la = 0;
   for (int i = 0; i < m; ++i) la += lam[i] * M->a[i];
   acc(1.0 - zeta - la);
   for (int i = 0; i < m; ++i) acc((v[3 + i] - M->a[i] * z - y[i] + s[i] - M->b[i]) / damp);
-  sum += v[1]; mx = std::max(mx, v[4 + MMAX]);
-  sum += v[2]; mx = std::max(mx, v[5 + MMAX]);
+  sum += v[1]; mx = std::max(mx, v[4 + m]);
+  sum += v[2]; mx = std::max(mx, v[5 + m]);
   for (int i = 0; i < m; ++i) acc(mu[i] * y[i] - M->eps);
   acc(zeta * z - M->eps);
   for (int i = 0; i < m; ++i) acc(lam[i] * s[i] - M->eps);
   return {std::sqrt(sum), mx};
 }
 
-bool mma_update_dev(tos_mma* M, hipStream_t st, const double* df, const double* dg, const double* g,
-                    std::function<void(int)> prof_mark = nullptr) {
-  (void)prof_mark;
+template <int MC>
+bool mma_update_m(tos_mma* M, hipStream_t st, const double* df, const double* dg, const double* g) {
   MmaVecs& V = M->V;
-  const int m = V.m;
+  constexpr int m = MC, CK = kkt_cols(MC), CP = point_cols(MC);
   MmaSmall S{};
   S.move = M->move;
-  constexpr unsigned KKT_MAX = (1u << (3 + MMAX)) | (1u << (4 + MMAX)) | (1u << (5 + MMAX));
   // p, q, b and the start point
   {
-    const double* v = mma_pass(M, st, k_mma_pq, m, 0u, V, df, dg, M->partial);
+    const double* v = mma_pass(M, st, k_mma_pq, m, 1, 0, V, df, dg, M->partial);
     for (int i = 0; i < m; ++i) M->b[i] = v[i] - g[i];
   }
   for (int i = 0; i < m; ++i) {
     M->y[i] = 1; M->lam[i] = 1; M->s[i] = 1; M->mu[i] = std::max(M->c[i] / 2, 1.0);
   }
   M->z = 1; M->zeta = 1; M->eps = 1;
-  for (int i = 0; i < m; ++i) S.lam[i] = M->lam[i];
-  hipLaunchKernelGGL(k_mma_plam, dim3(M->nb), dim3(256), 0, st, V, S);
-  LAUNCH_CHECK();
-  double lasterr = 0;
+  double lasterr = 0, move = 0;  // move: the accepted step still to be taken by the n-length vectors
   int nsub = 0;
   bool overflow = false;
   for (int lev = 0; lev < 6 && !overflow; ++lev) {
@@ -2488,23 +2484,27 @@ bool mma_update_dev(tos_mma* M, hipStream_t st, const double* df, const double* 
     int stays = 0;
     while (err > 0.9 * M->eps) {
       S.eps = M->eps;
-      constexpr int CA = MMAX + MMAX * MMAX + MMAX;
-      const double* v = mma_pass(M, st, k_mma_passA, CA, 0u, V, S, M->partial);
+      S.step = move;
+      for (int i = 0; i < m; ++i) S.lam[i] = M->lam[i];
+      double v[CP];
+      std::copy_n(mma_pass(M, st, k_mma_point<MC>, CP, CP, 3, V, S, M->partial), CP, v);
+      move = 0;
+      const double* kkt = v + m * m + m;  // its proxies: kkt[3 + i]
       // reduced (m+1) system (solveLinearSystem mma_t.cu:228-328), Gaussian elimination
       const int N1 = m + 1;
       double A[(MMAX + 1) * (MMAX + 1)] = {}, rhs[MMAX + 1], Dy[MMAX], dly[MMAX], dll[MMAX];
       for (int i = 0; i < m; ++i) {
         Dy[i] = M->d[i] + M->mu[i] / M->y[i];
         dly[i] = -(M->lam[i] + M->eps / M->y[i] - M->c[i] - M->d[i] * M->y[i]);
-        dll[i] = -(M->z * M->a[i] + M->y[i] + M->b[i] - M->eps / M->lam[i] - v[i]);
+        dll[i] = -(M->z * M->a[i] + M->y[i] + M->b[i] - M->eps / M->lam[i] - kkt[3 + i]);
       }
       double la = 0;
       for (int i = 0; i < m; ++i) la += M->lam[i] * M->a[i];
       const double dlz = -(la + M->eps / M->z - 1.0);
       for (int i = 0; i < m; ++i) {
         A[i * N1 + i] += M->s[i] / M->lam[i] + 1.0 / Dy[i];
-        for (int k = 0; k < m; ++k) A[i * N1 + k] += v[MMAX + i * MMAX + k];
-        rhs[i] = dll[i] + dly[i] / Dy[i] - v[MMAX + MMAX * MMAX + i];
+        for (int k = 0; k < m; ++k) A[i * N1 + k] += v[i * m + k];
+        rhs[i] = dll[i] + dly[i] / Dy[i] - v[m * m + i];
         A[i * N1 + m] = M->a[i];
         A[m * N1 + i] = M->a[i];
       }
@@ -2539,41 +2539,46 @@ bool mma_update_dev(tos_mma* M, hipStream_t st, const double* df, const double* 
       }
       const double dz = rhs[m];
       const double dzeta = M->eps / M->z - M->zeta - (M->zeta / M->z) * dz;
-      // step bound
-      const double* tv = mma_pass(M, st, k_mma_passB, 3, 7u, V, S, M->partial);
+      // step bound of the scalars; the device adds the vectors' and takes the step
       const double cf = 1.0 / 0.99;
-      double t3 = tv[2];
-      for (int i = 0; i < m; ++i) t3 = std::max(t3, -cf * dy[i] / M->y[i]);
-      t3 = std::max(t3, -cf * dz / M->z);
-      for (int i = 0; i < m; ++i) t3 = std::max(t3, -cf * dlam[i] / M->lam[i]);
-      for (int i = 0; i < m; ++i) t3 = std::max(t3, -cf * dmu[i] / M->mu[i]);
-      t3 = std::max(t3, -cf * dzeta / M->zeta);
-      for (int i = 0; i < m; ++i) t3 = std::max(t3, -cf * ds[i] / M->s[i]);
-      double step = 1.0 / std::max(std::max(tv[0], tv[1]), std::max(t3, 1.0));
-      // backtracking on the KKT 2-norm (search_step mma_t.cu:501-571)
-      for (int i = 0; i < m; ++i) S.lam[i] = M->lam[i];
-      const double* kv = mma_pass(M, st, k_mma_kkt<false>, 3 + MMAX + 3, KKT_MAX, V, S, M->partial);
-      const double old_err = mma_kkt_host(M, kv, M->y, M->lam, M->mu, M->s, M->z, M->zeta, 1.0).first;
-      double new_err = 1e30, new_inf = 1e30;
-      while (step > 1e-12 && new_err > old_err) {
+      double sb = 1.0;
+      for (int i = 0; i < m; ++i) sb = std::max(sb, -cf * dy[i] / M->y[i]);
+      sb = std::max(sb, -cf * dz / M->z);
+      for (int i = 0; i < m; ++i) sb = std::max(sb, -cf * dlam[i] / M->lam[i]);
+      for (int i = 0; i < m; ++i) sb = std::max(sb, -cf * dmu[i] / M->mu[i]);
+      sb = std::max(sb, -cf * dzeta / M->zeta);
+      for (int i = 0; i < m; ++i) sb = std::max(sb, -cf * ds[i] / M->s[i]);
+      hipLaunchKernelGGL(k_mma_direction<MC>, dim3(M->nb), dim3(256), 0, st, V, S, M->partial);
+      hipLaunchKernelGGL(k_mma_step, dim3(1), dim3(192), 0, st, (const double*)M->partial, M->nb, sb, M->red);
+      // backtracking on the KKT 2-norm (search_step mma_t.cu:501-571), kTrials steps at a time
+      const double old_err = mma_kkt_host(M, kkt, M->y, M->lam, M->mu, M->s, M->z, M->zeta, 1.0).first;
+      double new_err = 1e30, new_inf = 1e30, step = 1, scale = 1;
+      for (int k = 0; step > 1e-12 && new_err > old_err; ++k) {
+        if (k % kTrials == 0) {
+          hipLaunchKernelGGL(k_mma_trials<MC>, dim3(M->nb), dim3(256), 0, st, V, S, (const double*)(M->red + 3), scale,
+                             M->partial);
+          hipLaunchKernelGGL(k_mma_fold, dim3(kTrials * CK), dim3(64), 0, st, (const double*)M->partial, M->nb, CK, 3,
+                             M->red + 4);
+          LAUNCH_CHECK();
+          download(st, M->h_red, M->red, (4 + kTrials * CK) * sizeof(double));
+          step = M->h_red[3] * scale;
+          scale *= std::ldexp(1.0, -kTrials);
+          if (!(step > 1e-12)) break;
+        }
+        const double* kt = M->h_red + 4 + (k % kTrials) * CK;
         double ty[MMAX], tl[MMAX], tm[MMAX], ts[MMAX];
         for (int i = 0; i < m; ++i) {
           ty[i] = M->y[i] + dy[i] * step;
           tl[i] = M->lam[i] + dlam[i] * step;
           tm[i] = M->mu[i] + dmu[i] * step;
           ts[i] = M->s[i] + ds[i] * step;
-          S.lam[i] = tl[i];
         }
         const double tz = M->z + dz * step, tzeta = M->zeta + dzeta * step;
-        S.step = step;
-        const double* kt = mma_pass(M, st, k_mma_kkt<true>, 3 + MMAX + 3, KKT_MAX, V, S, M->partial);
         const auto e2 = mma_kkt_host(M, kt, ty, tl, tm, ts, tz, tzeta, damp);
         new_err = e2.first;
         new_inf = e2.second;
         if (new_err < old_err) {
-          std::swap(V.x, V.tx);
-          std::swap(V.xi, V.txi);
-          std::swap(V.eta, V.teta);
+          move = step;
           for (int i = 0; i < m; ++i) { M->y[i] = ty[i]; M->lam[i] = tl[i]; M->mu[i] = tm[i]; M->s[i] = ts[i]; }
           M->z = tz;
           M->zeta = tzeta;
@@ -2590,10 +2595,19 @@ bool mma_update_dev(tos_mma* M, hipStream_t st, const double* df, const double* 
     M->eps *= 0.1;
   }
   M->last_newton = nsub;
-  S.move = M->move;
-  const double* av = mma_pass(M, st, k_mma_asym, 1, 0u, V, S, M->partial);
+  S.step = move;  // the last accepted step
+  const double* av = mma_pass(M, st, k_mma_asym, 1, 1, 0, V, S, M->partial);
   if (std::sqrt(av[0]) < 1e-3) M->stop_counter++;
   return M->stop_counter > 10;
+}
+
+bool mma_update_dev(tos_mma* M, hipStream_t st, const double* df, const double* dg, const double* g) {
+  switch (M->V.m) {
+    case 1: return mma_update_m<1>(M, st, df, dg, g);
+    case 2: return mma_update_m<2>(M, st, df, dg, g);
+    case 3: return mma_update_m<3>(M, st, df, dg, g);
+    default: return mma_update_m<4>(M, st, df, dg, g);
+  }
 }
 
 template <class F>
@@ -4321,7 +4335,7 @@ TOS_EXPORT int tos_mma_create(int n, int m, const double* xmin, const double* xm
     M->move = move;
     for (int i = 0; i < MMAX; ++i) { M->a[i] = 0; M->c[i] = 10; M->d[i] = 1; }  // mma_t.h:206-207
     double** vecs[] = {&V.x, &V.xmin, &V.xmax, &V.L, &V.U, &V.alpha, &V.beta, &V.lastdx, &V.xi, &V.eta,
-                       &V.plam, &V.qlam, &V.curx, &V.Dx, &V.dlx, &V.dx, &V.dxi, &V.deta, &V.tx, &V.txi, &V.teta};
+                       &V.curx, &V.Dx, &V.dlx, &V.dx, &V.dxi, &V.deta};
     for (double** v : vecs) *v = malloc_mma<double>(M, n);
     V.p = malloc_mma<double>(M, (size_t)(m + 1) * n);
     V.q = malloc_mma<double>(M, (size_t)(m + 1) * n);
