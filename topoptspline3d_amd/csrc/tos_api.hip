@@ -1178,8 +1178,10 @@ void vcycle_level(Ctx& c, int l, const T* f, T* u, int pre, int post) {
   if (l == last && last > 0) {
     if (c.cn == 0) return;  // no unknowns on the coarsest level (u stays 0)
     Prof pr(c, P_COARSE);
-    hipLaunchKernelGGL((k_coarse_solve<T>), dim3(nblk((int64_t)c.cn * 64)), dim3(256), 0, c.stream, L.v,
-                       (const int64_t*)c.cidx, c.cn, coarse_inverse<T>(c), f, u);
+    auto k = c.cn <= 512 ? &k_coarse_solve<T, 8> : (c.cn <= 1024 ? &k_coarse_solve<T, 16> :
+             (c.cn <= 2048 ? &k_coarse_solve<T, 32> : &k_coarse_solve<T, 0>));
+    hipLaunchKernelGGL(k, dim3(nblk((int64_t)c.cn * 64)), dim3(256), 0, c.stream, L.v, (const int64_t*)c.cidx, c.cn,
+                       coarse_inverse<T>(c), f, u);
     LAUNCH_CHECK();
     return;
   }
