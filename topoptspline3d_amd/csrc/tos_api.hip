@@ -854,39 +854,46 @@ void gs_sweep_pairs(Ctx& c, T* u, const T* f, bool backward, bool from_zero) {
 // Fine-level FP32 sweep in four in-wave two-colour passes (k_fine_gs_pairw), each followed
 // by the copy of its deferred nodes; classes in colour order, forward (0,0) (1,0) (0,1)
 // (1,1) with the even-x colour first, backward the reverse with the odd-x colour first.
-void gs_sweep_pairw(Ctx& c, float* u, const float* f, bool backward, bool from_zero) {
+template <class T>
+void gs_sweep_pairw(Ctx& c, T* u, const T* f, bool backward, bool from_zero) {
   Level& L = c.L[0];
   const LevelView& v = L.v;
-  if (!L.pair_single && !L.ub32) L.ub32 = dalloc<float>(c, 3 * (size_t)v.NP);
-  float* ub = L.pair_single ? nullptr : L.ub32;  // rows of one segment: no deferred nodes
+  constexpr bool f32 = std::is_same<T, float>::value;
+  T* ub = nullptr;  // (rows of one segment: no deferred nodes)
+  if (!L.pair_single) {
+    if (f32 && !L.ub32) L.ub32 = dalloc<float>(c, 3 * (size_t)v.NP);
+    if (!f32 && !L.ubuf) L.ubuf = dalloc<double>(c, 3 * (size_t)v.NP);
+    ub = f32 ? (T*)L.ub32 : (T*)L.ubuf;
+  }
   const int P = backward ? 1 : 0;
   // the FCG's z.r and z.q from this sweep's final values (one sum per wave and pass)
   // (c.gsdots is sized by the solve before any capture: one zr and one zq per segment)
   int64_t nd = 0;
   for (int i = 0; i < 4; ++i) nd += L.n_segw[i][1];
-  const bool dots = backward && c.dots_last && c.dots_q && c.gsdots && c.gsdots_n == nd;
+  const bool dots = f32 && backward && c.dots_last && c.dots_q && c.gsdots && c.gsdots_n == nd;
   int64_t doff = 0;
   for (int i = 0; i < 4; ++i) {
     const int cls = backward ? 3 - i : i;
     const int n = L.n_segw[cls][P];
     if (!n) continue;
-    Prof pr(c, P_FINE_GS32);
+    Prof pr(c, f32 ? P_FINE_GS32 : P_FINE_GS64);
     const dim3 g((n + 3) / 4), b(256);
     const int4* sg = L.segw[cls][P];
     const uint8_t* fr = L.fre;
     if (dots) {
-      hipLaunchKernelGGL((k_fine_gs_pairw<float, true, -1, -1, true>), g, b, 0, c.stream, v, sg, n, fr, c.w32,
-                         c.Kc32, u, f, ub, c.dots_q, c.gsdots + doff, nd);
+      if constexpr (f32)
+        hipLaunchKernelGGL((k_fine_gs_pairw<float, true, -1, -1, true>), g, b, 0, c.stream, v, sg, n, fr, c.w32,
+                           c.Kc32, u, f, ub, c.dots_q, c.gsdots + doff, nd);
       doff += n;
     } else if (backward) {
-      hipLaunchKernelGGL((k_fine_gs_pairw<float, true, -1, -1>), g, b, 0, c.stream, v, sg, n, fr, c.w32, c.Kc32, u, f,
-                         ub, (const float*)nullptr, (double*)nullptr, (int64_t)0);
+      hipLaunchKernelGGL((k_fine_gs_pairw<T, true, -1, -1>), g, b, 0, c.stream, v, sg, n, fr, Prec<T>::w(c), Prec<T>::Ke(c), u, f,
+                         ub, (const T*)nullptr, (double*)nullptr, (int64_t)0);
     } else if (!from_zero) {
-      hipLaunchKernelGGL((k_fine_gs_pairw<float, false, -1, -1>), g, b, 0, c.stream, v, sg, n, fr, c.w32, c.Kc32, u,
-                         f, ub, (const float*)nullptr, (double*)nullptr, (int64_t)0);
+      hipLaunchKernelGGL((k_fine_gs_pairw<T, false, -1, -1>), g, b, 0, c.stream, v, sg, n, fr, Prec<T>::w(c), Prec<T>::Ke(c), u,
+                         f, ub, (const T*)nullptr, (double*)nullptr, (int64_t)0);
     } else {
-#define GO(A) hipLaunchKernelGGL((k_fine_gs_pairw<float, false, A, A + 1>), g, b, 0, c.stream, v, sg, n, fr, c.w32, \
-                                 c.Kc32, u, f, ub, (const float*)nullptr, (double*)nullptr, (int64_t)0)
+#define GO(A) hipLaunchKernelGGL((k_fine_gs_pairw<T, false, A, A + 1>), g, b, 0, c.stream, v, sg, n, fr, Prec<T>::w(c), \
+                                 Prec<T>::Ke(c), u, f, ub, (const T*)nullptr, (double*)nullptr, (int64_t)0)
       switch (cls) {
         case 0: GO(0); break;
         case 1: GO(2); break;
@@ -896,8 +903,8 @@ void gs_sweep_pairw(Ctx& c, float* u, const float* f, bool backward, bool from_z
 #undef GO
     }
     if (ub)
-      hipLaunchKernelGGL((k_fine_pairw_copy<float>), dim3(nblk(3 * (int64_t)n)), dim3(256), 0, c.stream, v, sg, n, fr,
-                         (const float*)ub, u);
+      hipLaunchKernelGGL((k_fine_pairw_copy<T>), dim3(nblk(3 * (int64_t)n)), dim3(256), 0, c.stream, v, sg, n, fr,
+                         (const T*)ub, u);
   }
   if (dots) c.dots_done = true;
   LAUNCH_CHECK();
@@ -991,11 +998,14 @@ void gs_sweep(Ctx& c, int l, T* u, const T* f, bool backward, bool from_zero = f
     gs_sweep_st_split<T>(c, l, u, f, backward, from_zero);
     return;
   }
-  if constexpr (std::is_same<T, float>::value) {
-    if (l == 0 && c.sweep_mode == 3) {
-      gs_sweep_pairw(c, u, f, backward, from_zero);
-      return;
-    }
+  // FP64 cycles pair two colours on levels of up to kPairBelow64 rows a class, where the launches'
+  // latency counts more than the occupancy that the pairs' 195 registers cost: ms per iteration
+  // with colour passes and pairs 5.12 / 4.69 at 24x12x12 (36 rows a class), 27.93 / 27.70 at
+  // 160x80x80 (1681)
+  constexpr int kPairBelow64 = 2048;
+  if (l == 0 && c.sweep_mode == 3 && (sizeof(T) == 4 || L.n_segw[0][0] < kPairBelow64)) {
+    gs_sweep_pairw<T>(c, u, f, backward, from_zero);
+    return;
   }
   // (FP32 cycles only: with FP64 values the paired kernel's registers halve its occupancy)
   if (std::is_same<T, float>::value && l > 0 && c.sweep_mode == 3 && L.pair_ok) {
