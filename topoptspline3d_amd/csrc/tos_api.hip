@@ -1542,8 +1542,18 @@ void fine_zero_sweep_b(Ctx& c, BatchState& B, float* u, const float* f, float* r
   LAUNCH_CHECK();
 }
 
-// one colour-ordered GS sweep of level l on the interleaved vectors
-void gs_b(Ctx& c, BatchState& B, int l, float* u, const float* f, bool backward) {
+// stencil level, colour `col` of a first forward sweep from zero
+template <int BS>
+void st_zero_colour_b(Ctx& c, BatchState& B, Level& L, int off, int nch, int col, float* u, const float* f) {
+#define GO(ZC) hipLaunchKernelGGL((k_st_gs_b<float, false, BS, ZC>), dim3(bgrid(nch, B.KP, BS)), dim3(BS), 0, c.stream, \
+                                  L.v, (const int4*)(L.cl_col + off), nch, 64 * (int64_t)off, B.K, B.KP,                \
+                                  (const float*)L.st32, L.NS, u, f)
+  TOS_COLOUR_SWITCH(col, GO);
+#undef GO
+}
+
+// one colour-ordered GS sweep of level l on the interleaved vectors (from_zero: stencil levels)
+void gs_b(Ctx& c, BatchState& B, int l, float* u, const float* f, bool backward, bool from_zero = false) {
   Level& L = c.L[l];
   const LevelView& v = L.v;
   const int bs = l == 0 ? B.bs_fine_gs : B.bs_st_gs[l];
@@ -1553,7 +1563,11 @@ void gs_b(Ctx& c, BatchState& B, int l, float* u, const float* f, bool backward)
     if (nch == 0) continue;
     const int4* cl = L.cl_col + off;
     const unsigned nb = bgrid(nch, B.KP, bs);
-    if (l == 0) {
+    if (l > 0 && from_zero) {
+#define GO(BS) st_zero_colour_b<BS>(c, B, L, off, nch, col, u, f)
+      TOS_BS_SWITCH(bs, GO)
+#undef GO
+    } else if (l == 0) {
 #define GO(BS)                                                                                                     \
   if (backward)                                                                                                    \
     hipLaunchKernelGGL((k_fine_gs_b<float, true, BS>), dim3(nb), dim3(BS), 0, c.stream, v, cl, nch, B.K, B.KP,     \
@@ -1655,14 +1669,16 @@ void vcycle_b(Ctx& c, BatchState& B, int l, const float* f, float* u, int pre, i
     for (int s = 0; s < post; ++s) gs_b(c, B, l, u, f, true);
     return;
   }
-  hipLaunchKernelGGL((k_zero_nodes_b<float, kVecBS>), dim3(bgrid(L.n_lin, B.KP, kVecBS)), dim3(kVecBS), 0, c.stream,
-                     (const int4*)L.cl_lin, L.n_lin, L.v.NP, B.K, B.KP, u);
+  // the first sweep of a stencil level starts from zero without clearing u
+  if (l == 0 || (l < last && pre == 0))
+    hipLaunchKernelGGL((k_zero_nodes_b<float, kVecBS>), dim3(bgrid(L.n_lin, B.KP, kVecBS)), dim3(kVecBS), 0, c.stream,
+                       (const int4*)L.cl_lin, L.n_lin, L.v.NP, B.K, B.KP, u);
   if (l == last) {
-    for (int s = 0; s < std::max(1, pre); ++s) gs_b(c, B, l, u, f, false);
+    for (int s = 0; s < std::max(1, pre); ++s) gs_b(c, B, l, u, f, false, l > 0 && s == 0);
     for (int s = 0; s < std::max(1, post); ++s) gs_b(c, B, l, u, f, true);
     return;
   }
-  for (int s = 0; s < pre; ++s) gs_b(c, B, l, u, f, false);
+  for (int s = 0; s < pre; ++s) gs_b(c, B, l, u, f, false, l > 0 && s == 0);
   resid_b(c, B, l, u, f, B.r32[l]);
   restrict_b(c, B, l, B.r32[l], B.f32[l + 1]);
   vcycle_b(c, B, l + 1, B.f32[l + 1], B.u32[l + 1], pre, post);
