@@ -189,17 +189,32 @@ __global__ __launch_bounds__(BS) void k_st_gs_b(LevelView L, const int4* __restr
   constexpr unsigned mask = nb_mask_of(ZC);
   load_nbhd_b<T, mask>(L, u, n.p, K, k, un);
   T s0 = 0, s1 = 0, s2 = 0;
-#pragma unroll
-  for (int q = 0; q < 27; ++q) {
-    if (q == 13 || !((mask >> q) & 1u)) continue;
-    const T u0 = un[q][0], u1 = un[q][1], u2 = un[q][2];
-    s0 = fma(S.get(slot, q, 0), u0, s0); s0 = fma(S.get(slot, q, 1), u1, s0); s0 = fma(S.get(slot, q, 2), u2, s0);
-    s1 = fma(S.get(slot, q, 3), u0, s1); s1 = fma(S.get(slot, q, 4), u1, s1); s1 = fma(S.get(slot, q, 5), u2, s1);
-    s2 = fma(S.get(slot, q, 6), u0, s2); s2 = fma(S.get(slot, q, 7), u1, s2); s2 = fma(S.get(slot, q, 8), u2, s2);
-  }
   T D[9];
+  // a node plane's blocks are loaded together before their products
 #pragma unroll
-  for (int e = 0; e < 9; ++e) D[e] = S.get(slot, 13, e);
+  for (int z = 0; z < 3; ++z) {
+    T A[9][9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i)
+      if ((mask >> (9 * z + i)) & 1u || 9 * z + i == 13)
+#pragma unroll
+        for (int e = 0; e < 9; ++e) A[i][e] = S.get(slot, 9 * z + i, e);
+    TOS_LOADS_DONE();
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+      const int q = 9 * z + i;
+      if (q == 13) {
+#pragma unroll
+        for (int e = 0; e < 9; ++e) D[e] = A[i][e];
+        continue;
+      }
+      if (!((mask >> q) & 1u)) continue;
+      const T u0 = un[q][0], u1 = un[q][1], u2 = un[q][2];
+      s0 = fma(A[i][0], u0, s0); s0 = fma(A[i][1], u1, s0); s0 = fma(A[i][2], u2, s0);
+      s1 = fma(A[i][3], u0, s1); s1 = fma(A[i][4], u1, s1); s1 = fma(A[i][5], u2, s1);
+      s2 = fma(A[i][6], u0, s2); s2 = fma(A[i][7], u1, s2); s2 = fma(A[i][8], u2, s2);
+    }
+  }
   const int64_t i0 = n.p * K + k;
   T v0 = ZC < 0 ? un[13][0] : T(0), v1 = ZC < 0 ? un[13][1] : T(0), v2 = ZC < 0 ? un[13][2] : T(0);
   block_relax<T, BACKWARD>(f[i0] - s0, f[cs + i0] - s1, f[2 * cs + i0] - s2, D, v0, v1, v2);
