@@ -158,12 +158,20 @@ __global__ __launch_bounds__(BS) void k_st_apply_b(LevelView L, const int4* __re
   load_nbhd_b(L, u, n.p, K, k, un);
   T a0 = 0, a1 = 0, a2 = 0;
 #pragma unroll
-  for (int q = 0; q < 27; ++q) {
-    const T u0 = un[q][0], u1 = un[q][1], u2 = un[q][2];
-    const int64_t sl = n.slot;
-    a0 = fma(S.get(sl, q, 0), u0, a0); a0 = fma(S.get(sl, q, 1), u1, a0); a0 = fma(S.get(sl, q, 2), u2, a0);
-    a1 = fma(S.get(sl, q, 3), u0, a1); a1 = fma(S.get(sl, q, 4), u1, a1); a1 = fma(S.get(sl, q, 5), u2, a1);
-    a2 = fma(S.get(sl, q, 6), u0, a2); a2 = fma(S.get(sl, q, 7), u1, a2); a2 = fma(S.get(sl, q, 8), u2, a2);
+  for (int z = 0; z < 3; ++z) {
+    T A[9][9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i)
+#pragma unroll
+      for (int e = 0; e < 9; ++e) A[i][e] = S.get(n.slot, 9 * z + i, e);
+    TOS_LOADS_DONE();
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+      const T u0 = un[9 * z + i][0], u1 = un[9 * z + i][1], u2 = un[9 * z + i][2];
+      a0 = fma(A[i][0], u0, a0); a0 = fma(A[i][1], u1, a0); a0 = fma(A[i][2], u2, a0);
+      a1 = fma(A[i][3], u0, a1); a1 = fma(A[i][4], u1, a1); a1 = fma(A[i][5], u2, a1);
+      a2 = fma(A[i][6], u0, a2); a2 = fma(A[i][7], u1, a2); a2 = fma(A[i][8], u2, a2);
+    }
   }
   const int64_t i0 = n.p * K + k;
   if (MODE == 0) {
