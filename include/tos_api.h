@@ -248,7 +248,7 @@ int tos_oc_update_projected(tos_ctx* ctx, double vgoal, double move, double damp
  * rho_out (float, may equal rho) out; inactive elements are copied through.  Runs on
  * `stream` (a hipStream_t, NULL = the null stream); g_out / steps_out (host, may be NULL)
  * make the call wait for the stream.  The bisection's partials and scalars live in one
- * fixed device array per GPU (2*8192 + 32 doubles), so n > TOS_NOALLOC_MAX_ELEMENTS
+ * fixed device array per GPU (2*8192 + 40 doubles), so n > TOS_NOALLOC_MAX_ELEMENTS
  * returns TOS_E_TOO_LARGE; calls that overlap on one GPU (other threads or streams)
  * share that array and race. */
 #define TOS_NOALLOC_MAX_ELEMENTS 67108864
