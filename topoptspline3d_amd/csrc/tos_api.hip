@@ -851,19 +851,21 @@ void gs_sweep_pairs(Ctx& c, T* u, const T* f, bool backward, bool from_zero) {
 // One colour-ordered sweep.  from_zero: u is 0 on entry (the first pre-smoothing sweep of a
 // V-cycle level), so colour c reads only the neighbours of colours < c; same updates as
 // a sweep over a zeroed u, without zeroing it first or reading the zeros.
-// Fine-level FP32 sweep in four in-wave two-colour passes (k_fine_gs_pairw), each followed
-// by the copy of its deferred nodes; classes in colour order, forward (0,0) (1,0) (0,1)
-// (1,1) with the even-x colour first, backward the reverse with the odd-x colour first.
+// Fine-level sweep in four in-wave two-colour passes (k_fine_gs_pairw), each followed
+// by the copy of its deferred nodes where rows span several segments (FP32 only); classes in
+// colour order, forward (0,0) (1,0) (0,1) (1,1) with the even-x colour first, backward the
+// reverse with the odd-x colour first.
 template <class T>
 void gs_sweep_pairw(Ctx& c, T* u, const T* f, bool backward, bool from_zero) {
   Level& L = c.L[0];
   const LevelView& v = L.v;
   constexpr bool f32 = std::is_same<T, float>::value;
-  T* ub = nullptr;  // (rows of one segment: no deferred nodes)
-  if (!L.pair_single) {
-    if (f32 && !L.ub32) L.ub32 = dalloc<float>(c, 3 * (size_t)v.NP);
-    if (!f32 && !L.ubuf) L.ubuf = dalloc<double>(c, 3 * (size_t)v.NP);
-    ub = f32 ? (T*)L.ub32 : (T*)L.ubuf;
+  T* ub = nullptr;  // (rows of one segment, as in every FP64 cycle that comes here: no deferred nodes)
+  if constexpr (f32) {
+    if (!L.pair_single) {
+      if (!L.ub32) L.ub32 = dalloc<float>(c, 3 * (size_t)v.NP);
+      ub = L.ub32;
+    }
   }
   const int P = backward ? 1 : 0;
   // the FCG's z.r and z.q from this sweep's final values (one sum per wave and pass)
@@ -902,9 +904,10 @@ void gs_sweep_pairw(Ctx& c, T* u, const T* f, bool backward, bool from_zero) {
       }
 #undef GO
     }
-    if (ub)
-      hipLaunchKernelGGL((k_fine_pairw_copy<T>), dim3(nblk(3 * (int64_t)n)), dim3(256), 0, c.stream, v, sg, n, fr,
-                         (const T*)ub, u);
+    if constexpr (f32)
+      if (ub)
+        hipLaunchKernelGGL((k_fine_pairw_copy<float>), dim3(nblk(3 * (int64_t)n)), dim3(256), 0, c.stream, v, sg, n,
+                           fr, (const float*)ub, u);
   }
   if (dots) c.dots_done = true;
   LAUNCH_CHECK();
@@ -998,12 +1001,13 @@ void gs_sweep(Ctx& c, int l, T* u, const T* f, bool backward, bool from_zero = f
     gs_sweep_st_split<T>(c, l, u, f, backward, from_zero);
     return;
   }
-  // FP64 cycles pair two colours on levels of up to kPairBelow64 rows a class, where the launches'
-  // latency counts more than the occupancy that the pairs' 195 registers cost: ms per iteration
-  // with colour passes and pairs 5.12 / 4.69 at 24x12x12 (36 rows a class), 27.93 / 27.70 at
-  // 160x80x80 (1681)
-  constexpr int kPairBelow64 = 2048;
-  if (l == 0 && c.sweep_mode == 3 && (sizeof(T) == 4 || L.n_segw[0][0] < kPairBelow64)) {
+  // FP64 cycles pair two colours where every row is one segment, so that no copy of deferred
+  // nodes follows a pass; with copies the pairs' launches and 195 registers (half the occupancy)
+  // cost what the saved passes gain.  ms of 20 FCG iterations with colour passes / pairs, rows of
+  // one segment: 3.68 / 3.31 at 24x12x12, 7.55 / 7.2 at 96x48x48, 18.8 / 17.9 at 120x100x100, 92.6 /
+  // 84.6 at 124x256x256, 77.5 / 75.2 at 30x300x300; of several: 9.97 / 10.2 at 400x30x30, 10.8 / 11.3
+  // at 128x64x64, 12.39 / 12.2 at 300x40x40, 16.0 / 15.9 at 160x80x80, 30.0 / 28.3 at 250x100x100
+  if (l == 0 && c.sweep_mode == 3 && (sizeof(T) == 4 || L.pair_single)) {
     gs_sweep_pairw<T>(c, u, f, backward, from_zero);
     return;
   }
