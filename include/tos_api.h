@@ -394,9 +394,11 @@ int tos_probe_element_mfma(tos_ctx* ctx, int reps, double* out);
  * workgroup per grid row relaxing the row's even-x colour then its odd-x colour; 3 = four
  * launches of two colours each, paired inside a wave (each lane relaxes a node of the
  * first colour, then the next node along x, using its neighbours' new values by lane
- * shuffles), also on the stored-stencil levels, FP32 cycles only (FP64 cycles use mode 0);
- * 3 is the default.  All perform exactly the same updates, so results are bit-identical
- * across modes. */
+ * shuffles); 3 is the default.  Modes 0 to 2 take eight colour passes on the stored-stencil
+ * levels, mode 3 takes four there too, except that FP64 cycles keep eight where a row needs more
+ * than one wave (125 free nodes along x always fit one), on any level, and on stored-stencil
+ * levels of 512 rows and more per parity class of (y, z).  All perform exactly the same updates
+ * in the same order of sums, so results are bit-identical across modes. */
 int tos_set_sweep_mode(tos_ctx* ctx, int mode);
 
 /* Storage precision of the Galerkin coarse operators built by tos_update_operator (no

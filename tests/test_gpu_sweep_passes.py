@@ -55,3 +55,16 @@ def test_fp64_fine_sweeps_pair_colours_on_rows_of_one_segment(hip, dims, paired)
     print(f"\n[passes] {dims}: mode 0 {n[0]}, mode 3 {n[3]}", flush=True)
     assert n[0] == 16
     assert n[3] == (8 if paired else 16)
+
+
+@pytest.mark.parametrize("precision", [0, 1, 2])
+def test_stencil_levels_with_few_rows_take_one_colour_a_pass_but_in_mode_3(hip, precision):
+    """Three levels, the second one a stored-stencil level of few rows, the third the coarsest
+    solve: two sweeps a cycle on the second, of eight passes in modes 0 to 2 and four in mode 3."""
+    c = context(hip, (40, 20, 24), n_levels=3)
+    n = []
+    for m in (0, 1, 2, 3):
+        c.set_sweep_mode(m)
+        n.append(passes(hip, c, precision, ("st_gs_f64", "st_gs_f32", "st_gs_f32_l1")))
+    print(f"\n[passes] precision {precision}: {n}", flush=True)
+    assert n == [16, 16, 16, 8]

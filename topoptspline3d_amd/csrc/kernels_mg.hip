@@ -1032,8 +1032,9 @@ __device__ __forceinline__ void st_row_add(const T (&A)[3][9], const T (&c)[4][3
 // colour's values.  ZERO: the first sweep from zero, where only rows of earlier classes hold
 // values.  Three waves, one per node plane: nine were no faster with FP16 and FP32 stencils and
 // slower with FP64, whose loads of a row they have no registers for (28 against 19 us a pass at
-// 420 rows of 80 nodes).
-template <class T, bool BACKWARD, bool ZERO, class ST>
+// 420 rows of 80 nodes).  PART: 0 both colours; 1 or 2 the first or the second alone, the second
+// with the first one's values from memory: the same sums, so the same values.
+template <class T, bool BACKWARD, bool ZERO, int PART, class ST>
 __global__ __launch_bounds__(192) void k_st_gs_split(LevelView L, const int4* __restrict__ seg,
                                                          const int* __restrict__ slotmap, ST st, T* __restrict__ u,
                                                          const T* __restrict__ f, int cls) {
@@ -1068,11 +1069,11 @@ __global__ __launch_bounds__(192) void k_st_gs_split(LevelView L, const int4* __
       T c[4][3];
       T A1[3][9], A2[3][9];
       load(r, c);
-      st_row_load(st, s1, r, A1);
-      st_row_load(st, s2, r, A2);
+      if constexpr (PART != 2) st_row_load(st, s1, r, A1);
+      if constexpr (PART != 1) st_row_load(st, s2, r, A2);
       TOS_LOADS_DONE();
-      st_row_add<T, 0>(A1, c, a);
-      st_row_add<T, 1>(A2, c, b);
+      if constexpr (PART != 2) st_row_add<T, 0>(A1, c, a);
+      if constexpr (PART != 1) st_row_add<T, 1>(A2, c, b);
     }
   };
   if (wv != 1) {
@@ -1086,8 +1087,12 @@ __global__ __launch_bounds__(192) void k_st_gs_split(LevelView L, const int4* __
     __syncthreads();
     return;
   }
-  T c[4][3] = {};  // the centre row (from zero: nothing there yet)
+  T c[4][3] = {};  // the centre row (from zero: nothing there yet but the first colour's values)
   if (!ZERO) load(4, c);
+  if (ZERO && PART == 2) {
+#pragma unroll
+    for (int e = 0; e < 3; ++e) c[1][e] = f1 ? u[e * L.NP + pa] : T(0);
+  }
   T A1[3][9], A2[3][9];
 #pragma unroll
   for (int j = 0; j < 3; ++j)
@@ -1122,8 +1127,9 @@ __global__ __launch_bounds__(192) void k_st_gs_split(LevelView L, const int4* __
     b[e] += part[0][3 + e][lane] + part[1][3 + e][lane];
   }
   T v[3] = {c[1][0], c[1][1], c[1][2]};
-  if (f1) block_relax<T, BACKWARD>(fma(fa[0], i1, -a[0]), fma(fa[1], i1, -a[1]), fma(fa[2], i1, -a[2]), A1[1], v[0],
-                                  v[1], v[2]);
+  if (PART != 2 && f1)
+    block_relax<T, BACKWARD>(fma(fa[0], i1, -a[0]), fma(fa[1], i1, -a[1]), fma(fa[2], i1, -a[2]), A1[1], v[0], v[1],
+                             v[2]);
   T w[3];
 #pragma unroll
   for (int e = 0; e < 3; ++e) w[e] = __shfl_down(v[e], 1, 64);  // the next lane's first-colour node
@@ -1132,12 +1138,13 @@ __global__ __launch_bounds__(192) void k_st_gs_split(LevelView L, const int4* __
 #pragma unroll
   for (int e = 0; e < 9; ++e) b[e / 3] = fma(A2[2][e], w[e % 3], b[e / 3]);
   T t[3] = {c[2][0], c[2][1], c[2][2]};
-  if (f2) block_relax<T, BACKWARD>(fma(fb[0], i2, -b[0]), fma(fb[1], i2, -b[1]), fma(fb[2], i2, -b[2]), A2[1], t[0],
-                                  t[1], t[2]);
+  if (PART != 1 && f2)
+    block_relax<T, BACKWARD>(fma(fb[0], i2, -b[0]), fma(fb[1], i2, -b[1]), fma(fb[2], i2, -b[2]), A2[1], t[0], t[1],
+                             t[2]);
 #pragma unroll
   for (int e = 0; e < 3; ++e) {
-    if (f1) u[e * L.NP + pa] = v[e];
-    if (f2) u[e * L.NP + pa + 1] = t[e];
+    if (PART != 2 && f1) u[e * L.NP + pa] = v[e];
+    if (PART != 1 && f2) u[e * L.NP + pa + 1] = t[e];
   }
 }
 

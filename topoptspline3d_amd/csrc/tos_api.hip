@@ -973,22 +973,33 @@ void gs_sweep_st_pairw(Ctx& c, int l, T* u, const T* f, bool backward, bool from
   LAUNCH_CHECK();
 }
 
-// Sweep of a level with few rows, two colours per pass and three waves per row
+// Sweep of a level with few rows, three waves per row: four passes of two colours in sweep mode
+// 3, eight of one in the other modes
+template <class T, int PART>
+void st_split_pass(Ctx& c, int l, int cls, T* u, const T* f, bool backward, bool from_zero) {
+  Level& L = c.L[l];
+  const int P = backward ? 1 : 0, n = L.n_segw[cls][P];
+  if (!n) return;
+  Prof pr(c, sizeof(T) == 8 ? P_ST_GS64 : (l == 1 ? P_ST_GS32_L1 : P_ST_GS32));
+  st_dispatch<T>(c, L, [&](auto st) {
+    using ST = decltype(st);
+    auto k = backward ? &k_st_gs_split<T, true, false, PART, ST>
+                      : (from_zero ? &k_st_gs_split<T, false, true, PART, ST> : &k_st_gs_split<T, false, false, PART, ST>);
+    hipLaunchKernelGGL(k, dim3(n), dim3(192), 0, c.stream, L.v, (const int4*)L.segw[cls][P], (const int*)L.slot, st, u,
+                       f, cls);
+  });
+}
+
 template <class T>
 void gs_sweep_st_split(Ctx& c, int l, T* u, const T* f, bool backward, bool from_zero) {
-  Level& L = c.L[l];
   for (int i = 0; i < 4; ++i) {
     const int cls = backward ? 3 - i : i;
-    const int n = L.n_segw[cls][backward ? 1 : 0];
-    if (!n) continue;
-    Prof pr(c, sizeof(T) == 8 ? P_ST_GS64 : (l == 1 ? P_ST_GS32_L1 : P_ST_GS32));
-    const int4* sg = L.segw[cls][backward ? 1 : 0];
-    st_dispatch<T>(c, L, [&](auto st) {
-      using ST = decltype(st);
-      auto k = backward ? &k_st_gs_split<T, true, false, ST>
-                        : (from_zero ? &k_st_gs_split<T, false, true, ST> : &k_st_gs_split<T, false, false, ST>);
-      hipLaunchKernelGGL(k, dim3(n), dim3(192), 0, c.stream, L.v, sg, (const int*)L.slot, st, u, f, cls);
-    });
+    if (c.sweep_mode == 3) {
+      st_split_pass<T, 0>(c, l, cls, u, f, backward, from_zero);
+    } else {
+      st_split_pass<T, 1>(c, l, cls, u, f, backward, from_zero);
+      st_split_pass<T, 2>(c, l, cls, u, f, backward, from_zero);
+    }
   }
   LAUNCH_CHECK();
 }
