@@ -915,11 +915,15 @@ void gs_sweep_pairw(Ctx& c, T* u, const T* f, bool backward, bool from_zero) {
 
 // Stored-stencil levels whose passes are short of waves take the kernels with several waves per
 // row (k_st_gs_split, k_st_apply_split), whatever the sweep mode and the cycle's precision.
-// Every row has to be one segment (at most 126 nodes), so that no node is deferred, and the
-// stencil below 4 GiB.  us a sweep pass / a residual, one wave and several: FP16 at 250 rows
-// 7.8 -> 5.7 / 7.5 -> 4.6, at 900 rows 12 against 13 / 9.3 (550 chunks) against 6.7 but 38
-// against 50 at 1900; FP32 at 290 rows 13.5 -> 9.0 / 6.8 -> 4.5; FP64 at 420 rows 2 x 17 (one
-// colour a pass) -> 19, at 110 rows 2 x 11.5 -> 7.5 / 14.5 -> 7.8, at 880 chunks 16 against 23.
+// Every row has to be one segment (125 nodes always are), so that no node is deferred, and the
+// stencil below 4 GiB.  One limit, on rows of the even (y, z) class for sweeps and on chunks for the
+// residual, lies below the crossings of all three precisions.  us with one wave -> several of a
+// forward sweep from zero and a backward one, over rows of 20 to 120 nodes: FP16 58 -> 44 at 256
+// rows, 69 -> 60 at 484, 81 -> 78 at 676, 102 -> 104 at 961; FP32 90 -> 47, 112 -> 88, 149 -> 129,
+// 187 -> 178; FP64 (one colour a pass) 183 -> 67, 235 -> 139, 252 -> 193, 286 -> 259.  Of a residual:
+// FP16 6.0 -> 3.9 at 242 chunks, 6.5 -> 5.4 at 392, 6.4 -> 5.5 at 512, 6.5 -> 7.8 at 800; FP32 7.0 ->
+// 5.0, 8.8 -> 7.2, 8.6 -> 7.6, 8.8 -> 13.1; FP64 12.4 -> 7.1, 14.1 -> 11.1, 14.2 -> 13.0 (11.5 -> 13.0
+// with rows of 20), 14.9 -> 20.6.
 constexpr int kSplitBelow = 512;
 inline bool small_stencil(const Level& L) { return L.NS * 243 * (int64_t)sizeof(double) < (int64_t)1 << 32; }
 inline bool gs_split(const Level& L) {
