@@ -40,3 +40,37 @@ def test_a_box_without_surface_points(hip):  # noqa: F811
         s = c.surface_constraints(cells=20, beta=8.0)
         assert s["n_points"] == 0
         assert not np.any(c.coeff_sens(2)) and not np.any(c.coeff_sens(3))
+
+
+def plane(nx, ny, nz, param):
+    """coefficients of a tilted plane surface, uniform lattice"""
+    ncx, ncy, ncz = (nx + param - 1) // param + 1, (ny + param - 1) // param + 1, (nz + param - 1) // param + 1
+    k, j, i = np.meshgrid(np.arange(ncz), np.arange(ncy), np.arange(ncx), indexing="ij")
+    return np.clip(0.5 + 0.9 * (k / ncz + 0.25 * i / ncx - 0.6), 0.01, 1).astype(np.float32).ravel()
+
+
+def cantilever_box(*dims):
+    from topoptspline3d_amd.domains import cantilever
+    return cantilever(*dims)
+
+
+def test_memory_follows_the_occupied_cells(hip):  # noqa: F811
+    """Order 8 (8 KB of sums per occupied cell), a plane through 45 x 33 x 33 coefficients: two
+    thousand occupied cells of 5e4, 1e4 points.  Lattice and points need 400 MB at 84 cells; sums
+    for as many cells as points would add 160 MB.  Other lattice sizes replace the buffers."""
+    import torch
+    from topoptspline3d_amd.context import Context
+    solid, support, _ = cantilever_box(88, 64, 64)
+    c = Context(hip, solid, support)
+    c.set_material(1e6, 0.4, 3.0, 1e-3)
+    c.spline_init(1, 8, 2)
+    c.set_coeffs(plane(88, 64, 64, 2))
+    used = []
+    free0 = torch.cuda.mem_get_info()[0]
+    for cells in (84, 40, 84, 40, 84):
+        s = c.surface_constraints(cells=cells, beta=8.0)
+        used.append((free0 - torch.cuda.mem_get_info()[0]) >> 20)
+        print(f"\n[surface] cells {cells}: {s['n_points']} points, {used[-1]} MB", flush=True)
+    nl = 86 ** 3
+    assert used[0] <= (592 * nl + 2400 * s["n_points"] >> 20) + 60
+    assert used[4] <= used[0] + 40 and used[3] < used[0]

@@ -79,6 +79,23 @@ T* dalloc(Ctx& c, size_t n) {
   return (T*)raw_alloc(c.allocs, c.stream, n * sizeof(T));
 }
 
+// gives an allocation of the context back (hipFree waits for the work that uses it)
+template <class T>
+void dfree(Ctx& c, T*& p) {
+  if (!p) return;
+  ++c.alloc_epoch;
+  c.allocs.erase(std::find(c.allocs.begin(), c.allocs.end(), (void*)p));
+  HIPCHK(hipFree(p));
+  p = nullptr;
+}
+
+// replaces an allocation of the context by one of n elements
+template <class T>
+void regrow(Ctx& c, T*& p, size_t n) {
+  dfree(c, p);
+  p = dalloc<T>(c, n);
+}
+
 inline unsigned nblk(int64_t n, int bs = 256) { return (unsigned)((n + bs - 1) / bs); }
 
 // launch shape of the stored-stencil paired GS (one wave per segment, no block-wide
@@ -3950,10 +3967,11 @@ TOS_EXPORT int tos_spline_init(tos_ctx* c, int mode, int order, int param) {
     for (int a = 0; a < 3; ++a) T[a] = spline_table(mode, order, param, dims[a], c->h);
     c->sp_mode = mode; c->sp_order = order; c->sp_param = param;
     // the surface-constraint state belongs to the previous spline (knots, coefficient count)
-    for (double*& U : c->sf_knots) U = nullptr;
-    c->sscsens = c->dripcsens = nullptr;
     c->sf_ncoef = 0;
     c->sf_valid = false;
+    for (double*& U : c->sf_knots) dfree(*c, U);
+    dfree(*c, c->sscsens);
+    dfree(*c, c->dripcsens);
     for (int a = 0; a < 3; ++a) {
       c->nc[a] = T[a].nc;
       c->sp_idx[a] = dalloc<int>(*c, T[a].idx.size());
@@ -4169,36 +4187,39 @@ TOS_EXPORT int tos_surface_constraints(tos_ctx* c, const tos_surface_opts* o, to
     const int NB = o->cells + 2;
     const int64_t nl = (int64_t)NB * NB * NB, cap = 3 * nl;
     const size_t ncoef = (size_t)C.nc[0] * C.nc[1] * C.nc[2];
+    // (outgrown buffers are given back; the sizes stand for the buffers only once all are there)
     if (C.sf_cells != o->cells) {  // lattice buffers for this lattice size
-      C.sf_val = dalloc<double>(C, nl);
-      C.sf_cnt = dalloc<int>(C, nl);
-      C.sf_off = dalloc<int>(C, nl + 1);
+      C.sf_cells = 0;
+      C.sf_valid = false;
+      regrow(C, C.sf_val, nl);
+      regrow(C, C.sf_cnt, nl);
+      regrow(C, C.sf_off, nl + 1);
       const int64_t nsb = (nl + kSfScanBlock - 1) / kSfScanBlock;
-      C.sf_bsum = dalloc<int>(C, nsb);
-      C.sf_boff = dalloc<int>(C, nsb + 1);
-      C.sf_tab_i = dalloc<int>(C, 3 * 8 * (int64_t)NB);
-      C.sf_tab_v = dalloc<double>(C, 3 * 8 * (int64_t)NB);
-      C.sf_tab_ok = dalloc<uint8_t>(C, 3 * (int64_t)NB);
-      C.sf_pts = dalloc<double>(C, 3 * cap);
-      C.sf_grad = dalloc<double>(C, 3 * cap);
-      C.sf_hess = dalloc<double>(C, 6 * cap);
-      C.sf_nrm = dalloc<double>(C, 3 * cap);
-      C.sf_wss = dalloc<double>(C, 3 * cap);
-      C.sf_wdr = dalloc<double>(C, 6 * cap);
+      regrow(C, C.sf_bsum, nsb);
+      regrow(C, C.sf_boff, nsb + 1);
+      regrow(C, C.sf_tab_i, 3 * 8 * (int64_t)NB);
+      regrow(C, C.sf_tab_v, 3 * 8 * (int64_t)NB);
+      regrow(C, C.sf_tab_ok, 3 * (int64_t)NB);
+      regrow(C, C.sf_pts, 3 * cap);
+      regrow(C, C.sf_grad, 3 * cap);
+      regrow(C, C.sf_hess, 6 * cap);
+      regrow(C, C.sf_nrm, 3 * cap);
+      regrow(C, C.sf_wss, 3 * cap);
+      regrow(C, C.sf_wdr, 6 * cap);
       C.sf_cells = o->cells;
     }
     if (C.sf_ncoef != (int64_t)ncoef) {  // per-coefficient (and per-knot-cell) buffers
-      C.sscsens = dalloc<float>(C, ncoef);
-      C.dripcsens = dalloc<float>(C, ncoef);
-      C.sf_ccnt = dalloc<int>(C, ncoef);
-      C.sf_cstart = dalloc<int>(C, ncoef + 1);
+      C.sf_ncoef = 0;
+      regrow(C, C.sscsens, ncoef);
+      regrow(C, C.dripcsens, ncoef);
+      regrow(C, C.sf_ccnt, ncoef);
+      regrow(C, C.sf_cstart, ncoef + 1);
       const int64_t nsb = ((int64_t)ncoef + kSfScanBlock - 1) / kSfScanBlock;
-      C.sf_cbsum = dalloc<int>(C, nsb);
-      C.sf_cboff = dalloc<int>(C, nsb + 1);
-      C.sf_slot = dalloc<int>(C, ncoef);
-      C.sf_scell = dalloc<int>(C, ncoef);
-      C.sf_nslot = dalloc<int>(C, 1);
-      C.sf_touch = dalloc<uint8_t>(C, ncoef);
+      regrow(C, C.sf_cbsum, nsb);
+      regrow(C, C.sf_cboff, nsb + 1);
+      regrow(C, C.sf_slot, ncoef);
+      regrow(C, C.sf_scell, ncoef);
+      regrow(C, C.sf_touch, ncoef);
       C.sf_ncoef = (int64_t)ncoef;
     }
     {  // all coefficients equal: no surface; the driver's constants (utils/test_utils.cpp:1106-1113)
@@ -4269,8 +4290,42 @@ TOS_EXPORT int tos_surface_constraints(tos_ctx* c, const tos_surface_opts* o, to
                        C.partial);
     hipLaunchKernelGGL(k_sf_fold, dim3(1), dim3(256), 0, C.stream, (const double*)C.partial, (int)nbp, 3, S_TMP0,
                        C.scal);
+    // points grouped by knot cell: count, scan, slots; their number comes with the values below
+    if (C.sf_bcap < std::max<int64_t>(n, 1)) {
+      const int64_t bcap = std::max<int64_t>(n, 1024) * 2;
+      C.sf_bcap = 0;
+      regrow(C, C.sf_bidx, 3 * bcap);
+      regrow(C, C.sf_bN, 72 * bcap);
+      regrow(C, C.sf_key, bcap);
+      regrow(C, C.sf_list, bcap);
+      regrow(C, C.sf_sorted, bcap);
+      C.sf_bcap = bcap;
+    }
+    const int64_t nc64 = (int64_t)ncoef, kk = (int64_t)C.sp_order * C.sp_order * C.sp_order;
+    int* const nslot = (int*)(C.scal + S_SLOTS);
+    hipLaunchKernelGGL(k_zero<int>, dim3(nblk(nc64)), dim3(256), 0, C.stream, C.sf_ccnt, nc64);
+    if (n) {
+      hipLaunchKernelGGL(k_sf_basis, dim3(nblk(3 * n)), dim3(256), 0, C.stream, S, n, (const double*)C.sf_pts,
+                         C.sf_bidx, C.sf_bN);
+      hipLaunchKernelGGL(k_sf_cell_count, dim3(nblk(n)), dim3(256), 0, C.stream, n, C.nc[0], C.nc[1],
+                         (const int*)C.sf_bidx, C.sf_key, C.sf_ccnt);
+    }
+    {
+      const unsigned nsb = (unsigned)((nc64 + kSfScanBlock - 1) / kSfScanBlock);
+      hipLaunchKernelGGL(k_sf_scan_blocks, dim3(nsb), dim3(1024), 0, C.stream, (const int*)C.sf_ccnt, nc64,
+                         C.sf_cbsum);
+      hipLaunchKernelGGL(k_sf_scan, dim3(1), dim3(1024), 0, C.stream, (const int*)C.sf_cbsum, (int64_t)nsb,
+                         C.sf_cboff);
+      hipLaunchKernelGGL(k_sf_scan_apply, dim3(nsb), dim3(1024), 0, C.stream, (const int*)C.sf_ccnt, nc64,
+                         (const int*)C.sf_cboff, C.sf_cstart);
+    }
+    hipLaunchKernelGGL(k_zero<int>, dim3(1), dim3(256), 0, C.stream, nslot, (int64_t)1);
+    hipLaunchKernelGGL(k_sf_cell_slots, dim3(nblk(nc64)), dim3(256), 0, C.stream, nc64, (const int*)C.sf_ccnt, nslot,
+                       C.sf_slot, C.sf_scell);
     LAUNCH_CHECK();
     const double* hs = read_scal(C);
+    int slots = 0;
+    std::memcpy(&slots, hs + S_SLOTS, sizeof(int));
     const double dir = hs[S_TMP3] > 0 ? 1.0 : -1.0;
     const double ss_sum = hs[S_TMP0], dr_sum = hs[S_TMP1], n_down = hs[S_TMP2];
     // global values (global_selfsupp_constraint grid/Grid.cu:6101-6145, global_drip_constraint
@@ -4292,51 +4347,22 @@ TOS_EXPORT int tos_surface_constraints(tos_ctx* c, const tos_surface_opts* o, to
       dr_val = o->drip_mode <= 1 ? -1.0 : dr_sum / cnt_dr;
       dr_fac = o->drip_mode >= 6 ? 1.0 / cnt_dr : 0.0;
     }
-    if (C.sf_bcap < std::max<int64_t>(n, 1)) {
-      C.sf_bcap = std::max<int64_t>(n, 1024) * 2;
-      C.sf_bidx = dalloc<int>(C, 3 * C.sf_bcap);
-      C.sf_bN = dalloc<double>(C, 72 * C.sf_bcap);
-      C.sf_key = dalloc<int>(C, C.sf_bcap);
-      C.sf_list = dalloc<int>(C, C.sf_bcap);
-      C.sf_sorted = dalloc<int>(C, C.sf_bcap);
+    // the points of a cell in order, the sums of every occupied cell, and the gather over the cells
+    if (C.sf_pcap < 2 * kk * slots) {
+      const int64_t pcap = 2 * kk * (slots + slots / 2);
+      C.sf_pcap = 0;
+      regrow(C, C.sf_part, pcap);
+      C.sf_pcap = pcap;
     }
-    // points grouped by knot cell (count, scan, fill, per-cell sort), the sums of every
-    // occupied cell (at most one cell per point), then the gather over the cells
-    const int64_t nc64 = (int64_t)ncoef, kk = (int64_t)C.sp_order * C.sp_order * C.sp_order;
-    const int64_t max_slots = std::min<int64_t>(n, nc64);
-    if (C.sf_pcap < 2 * kk * max_slots) {
-      C.sf_pcap = std::min<int64_t>(2 * max_slots, nc64) * 2 * kk;
-      C.sf_part = dalloc<double>(C, C.sf_pcap);
-    }
-    hipLaunchKernelGGL(k_zero<int>, dim3(nblk(nc64)), dim3(256), 0, C.stream, C.sf_ccnt, nc64);
-    if (n) {
-      hipLaunchKernelGGL(k_sf_basis, dim3(nblk(3 * n)), dim3(256), 0, C.stream, S, n, (const double*)C.sf_pts,
-                         C.sf_bidx, C.sf_bN);
-      hipLaunchKernelGGL(k_sf_cell_count, dim3(nblk(n)), dim3(256), 0, C.stream, n, C.nc[0], C.nc[1],
-                         (const int*)C.sf_bidx, C.sf_key, C.sf_ccnt);
-    }
-    {
-      const unsigned nsb = (unsigned)((nc64 + kSfScanBlock - 1) / kSfScanBlock);
-      hipLaunchKernelGGL(k_sf_scan_blocks, dim3(nsb), dim3(1024), 0, C.stream, (const int*)C.sf_ccnt, nc64,
-                         C.sf_cbsum);
-      hipLaunchKernelGGL(k_sf_scan, dim3(1), dim3(1024), 0, C.stream, (const int*)C.sf_cbsum, (int64_t)nsb,
-                         C.sf_cboff);
-      hipLaunchKernelGGL(k_sf_scan_apply, dim3(nsb), dim3(1024), 0, C.stream, (const int*)C.sf_ccnt, nc64,
-                         (const int*)C.sf_cboff, C.sf_cstart);
-    }
-    hipLaunchKernelGGL(k_zero<int>, dim3(1), dim3(256), 0, C.stream, C.sf_nslot, (int64_t)1);
-    hipLaunchKernelGGL(k_sf_cell_slots, dim3(nblk(nc64)), dim3(256), 0, C.stream, nc64, (const int*)C.sf_ccnt,
-                       C.sf_nslot, C.sf_slot, C.sf_scell);
     hipLaunchKernelGGL(k_zero<int>, dim3(nblk(nc64)), dim3(256), 0, C.stream, C.sf_ccnt, nc64);
     hipLaunchKernelGGL(k_zero<uint8_t>, dim3(nblk(nc64)), dim3(256), 0, C.stream, C.sf_touch, nc64);
-    if (n) {
+    if (slots) {
       hipLaunchKernelGGL(k_sf_cell_fill, dim3(nblk(n)), dim3(256), 0, C.stream, n, (const int*)C.sf_key,
                          (const int*)C.sf_cstart, C.sf_ccnt, C.sf_list);
-      hipLaunchKernelGGL(k_sf_cell_sort, dim3(nblk(64 * max_slots)), dim3(256), 0, C.stream, (const int*)C.sf_nslot,
+      hipLaunchKernelGGL(k_sf_cell_sort, dim3(nblk(64 * (int64_t)slots)), dim3(256), 0, C.stream, (const int*)nslot,
                          (const int*)C.sf_scell, (const int*)C.sf_cstart, (const int*)C.sf_list, C.sf_sorted);
-      hipLaunchKernelGGL(k_sf_cell_grad, dim3(nblk(64 * max_slots)), dim3(256), 0, C.stream, S,
-                         (const int*)C.sf_nslot, (const int*)C.sf_scell, (const int*)C.sf_cstart,
-                         (const int*)C.sf_sorted, (const double*)C.sf_bN, (const double*)C.sf_wss,
+      hipLaunchKernelGGL(k_sf_cell_grad, dim3(nblk(64 * (int64_t)slots)), dim3(256), 0, C.stream, S, (const int*)nslot,
+                         (const int*)C.sf_scell, (const int*)C.sf_cstart, (const int*)C.sf_sorted, (const double*)C.sf_bN, (const double*)C.sf_wss,
                          (const double*)C.sf_wdr, C.sf_part, C.sf_touch);
     }
     hipLaunchKernelGGL(k_sf_grad, dim3(nblk((nc64 + kSfGradC - 1) / kSfGradC * 64)), dim3(256), 0, C.stream, S, nc64,

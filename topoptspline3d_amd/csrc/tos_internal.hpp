@@ -257,7 +257,6 @@ struct Ctx {
   int* sf_list = nullptr;    // points grouped by knot cell, in arrival and in point order
   int* sf_sorted = nullptr;
   int *sf_slot = nullptr, *sf_scell = nullptr;  // occupied cells: slot of a cell (-1 empty), cell of a slot
-  int* sf_nslot = nullptr;
   uint8_t* sf_touch = nullptr;                  // coefficients reached by any point
   double* sf_part = nullptr;                    // k^3 pairs of gradient sums per occupied cell
   int64_t sf_pcap = 0;                          // doubles in sf_part
@@ -321,6 +320,7 @@ enum {
   S_RIG0,                            // 6 slots: R^T v of a rigid-motion projection
   S_AH0 = S_RIG0 + 6,                // 4 slots: alpha of the directions in the four direction
                                      // buffers of the precision-3 FCG
+  S_SLOTS = S_AH0 + 4,               // an int: number of occupied knot cells (k_sf_cell_slots)
   S_COUNT = 40
 };
-static_assert(S_AH0 + 4 <= S_COUNT, "scalar slots");
+static_assert(S_SLOTS < S_COUNT, "scalar slots");
