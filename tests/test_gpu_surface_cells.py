@@ -49,6 +49,47 @@ def plane(nx, ny, nz, param):
     return np.clip(0.5 + 0.9 * (k / ncz + 0.25 * i / ncx - 0.6), 0.01, 1).astype(np.float32).ravel()
 
 
+@pytest.mark.parametrize("param,cells", [(16, (8, 9, 12, 48)), (6, (40, 64))])
+def test_cells_of_more_points_than_a_slot(hip, param, cells):  # noqa: F811
+    """Knot cells of less than one, one and a few, and up to some thirty slots of 128 points: the
+    point order within a cell and the sums over a cell's slots."""
+    nx, ny, nz = 24, 16, 20
+    (o, g), n = pair(hip, nx, ny, nz, 1, 4, param)
+    cf = np.random.default_rng(param).uniform(0.05, 1.0, n).astype(np.float32)
+    for c in (o, g):
+        c.set_coeffs(cf)
+    for m in cells:
+        so, sg = (c.surface_constraints(cells=m, beta=8.0, ss_mode=4, drip_mode=7, drip_beta=4.0, drip_mu=2.0,
+                                        drip_beta_scale=1.0) for c in (o, g))
+        print(param, m, sg, flush=True)
+        assert so["n_points"] == sg["n_points"] > 0
+        first = [g.coeff_sens(w).copy() for w in (2, 3)]
+        for which in (2, 3):
+            go = o.coeff_sens(which)
+            assert np.abs(first[which - 2] - go).max() <= 1e-5 * max(np.abs(go).max(), 1e-30), (m, which)
+        g.surface_constraints(cells=m, beta=8.0, ss_mode=4, drip_mode=7, drip_beta=4.0, drip_mu=2.0,
+                              drip_beta_scale=1.0)
+        assert all(np.array_equal(g.coeff_sens(w), first[w - 2]) for w in (2, 3)), m
+
+
+def test_a_lattice_much_finer_than_the_knots_takes_no_serial_chain(hip):  # noqa: F811
+    """2e5 points in a few knot cells: some milliseconds; a chain over a cell's points, or over
+    their pairs in one wavefront, takes seconds."""
+    import time
+    solid, support, _ = cantilever_box(32, 20, 20)
+    from topoptspline3d_amd.context import Context
+    c = Context(hip, solid, support)
+    c.set_material(1e6, 0.4, 3.0, 1e-3)
+    n = c.spline_init(1, 4, 16)
+    c.set_coeffs(np.random.default_rng(3).uniform(0.05, 1.0, n).astype(np.float32))
+    c.surface_constraints(cells=256, beta=8.0)
+    t = time.perf_counter()
+    s = c.surface_constraints(cells=256, beta=8.0)
+    t = time.perf_counter() - t
+    print(f"\n[surface] {s['n_points']} points, {t * 1e3:.1f} ms", flush=True)
+    assert s["n_points"] > 100000 and t < 1.0
+
+
 def cantilever_box(*dims):
     from topoptspline3d_amd.domains import cantilever
     return cantilever(*dims)

@@ -525,21 +525,26 @@ __global__ void k_sf_cell_count(int64_t n, int ncx, int ncy, const int* __restri
   key[t] = c;
 }
 
-// The cells that hold points get consecutive slots: slot[cell] (-1: empty), scell[slot].
-// Which slot a cell gets depends on scheduling; it only names a place in `part` below.
+// The cells that hold points get slots, one per kSfChunk points of the cell, consecutive ones:
+// slot[cell] = (first, end) of them, scell[slot] the cell.  Which slots a cell gets depends on
+// scheduling; they only name places in `part` below.
+constexpr int kSfChunk = 128;
 __global__ void k_sf_cell_slots(int64_t ncell, const int* __restrict__ cnt, int* __restrict__ nslot,
-                                int* __restrict__ slot, int* __restrict__ scell) {
+                                int2* __restrict__ slot, int* __restrict__ scell) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const bool has = c < ncell && cnt[c] > 0;
-  const unsigned long long m = __ballot(has);
-  const int lane = threadIdx.x & 63;
+  const int nch = c < ncell ? (cnt[c] + kSfChunk - 1) / kSfChunk : 0, lane = threadIdx.x & 63;
+  int end = nch;  // slots of the wave's cells up to this one
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(end, o, 64);
+    if (lane >= o) end += v;
+  }
   int base = 0;
-  if (m && lane == __ffsll((unsigned long long)m) - 1) base = atomicAdd(nslot, __popcll(m));
-  if (m) base = __shfl(base, __ffsll((unsigned long long)m) - 1, 64);
+  if (lane == 63 && end) base = atomicAdd(nslot, end);
+  base = __shfl(base, 63, 64);
   if (c >= ncell) return;
-  const int s = base + __popcll(m & ((1ull << lane) - 1));
-  slot[c] = has ? s : -1;
-  if (has) scell[s] = (int)c;
+  const int s = base + end - nch;
+  slot[c] = make_int2(s, s + nch);
+  for (int q = 0; q < nch; ++q) scell[s + q] = (int)c;
 }
 
 // list[start[cell] ..) = the cell's points; cur (zeroed) hands out the slots in arrival
@@ -551,37 +556,53 @@ __global__ void k_sf_cell_fill(int64_t n, const int* __restrict__ key, const int
   list[start[key[t]] + atomicAdd(&cur[key[t]], 1)] = (int)t;
 }
 
-// One wavefront per occupied cell: every lane ranks its points among the cell's (distinct)
-// points and stores them there.  A lattice finer than the knots puts hundreds of points in
-// a cell: one thread per cell sorting in place took 6.7 ms on 128 cells over 128 x 64 x 64
-// voxels, this 0.08 ms.
+// One wavefront per slot: every lane ranks two of the slot's points among the cell's (distinct)
+// points, 64 of them at a time from a register that the lanes read in turn, and stores them at
+// their ranks.  The work is quadratic in the points of a cell, but spread over the cell's slots:
+// a lattice much finer than the knots puts 1e4 and more points in a cell, where one wavefront per
+// cell was a serial chain (ms of the call, 256 cells over 32x20x20 voxels: 520 -> 5.4 with 6
+// voxels per knot, 27 000 -> 15 with 16).
 __global__ __launch_bounds__(256) void k_sf_cell_sort(const int* __restrict__ nslot, const int* __restrict__ scell,
-                                                      const int* __restrict__ start, const int* __restrict__ list,
-                                                      int* __restrict__ sorted) {
+                                                      const int2* __restrict__ slot, const int* __restrict__ start,
+                                                      const int* __restrict__ list, int* __restrict__ sorted) {
   const int s = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * 256 + threadIdx.x) >> 6));
   if (s >= *nslot) return;  // whole wavefronts
-  const int c = scell[s], b = start[c], e = start[c + 1];
-  for (int i = b + (int)(threadIdx.x & 63); i < e; i += 64) {
-    const int v = list[i];
-    int r = b;
-    for (int j = b; j < e; ++j) r += list[j] < v ? 1 : 0;
-    sorted[r] = v;
+  const int c = scell[s], b = start[c], e = start[c + 1], lane = threadIdx.x & 63;
+  const int i0 = b + (s - slot[c].x) * kSfChunk + lane, i1 = i0 + 64;
+  const int v0 = i0 < e ? list[i0] : 0, v1 = i1 < e ? list[i1] : 0;
+  int r0 = b, r1 = b;
+  int next = b + lane < e ? list[b + lane] : INT_MAX;  // (INT_MAX ranks below no point)
+  for (int j = b; j < e; j += 64) {
+    const int t = next;
+    next = j + 64 + lane < e ? list[j + 64 + lane] : INT_MAX;
+    const int m = min(64, e - j);  // (a multiple of 8 are read)
+    for (int k = 0; k < m; k += 8) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int x = __builtin_amdgcn_readlane(t, k + i);
+        r0 += x < v0 ? 1 : 0;
+        r1 += x < v1 ? 1 : 0;
+      }
+    }
   }
+  if (i0 < e) sorted[r0] = v0;
+  if (i1 < e) sorted[r1] = v1;
 }
 
-// part[(slot k^3 + w) 2 ..) = the sums over a cell's points of w . (basis derivatives) for
+// part[(slot k^3 + w) 2 ..) = the sums over a slot's points of w . (basis derivatives) for
 // the coefficient at offset w = i + k (j + k l) of the cell's block, self-support and drip.
-// One wavefront per occupied cell, lane = offset (all 64 busy at order 4), points in
-// ascending order; touch[c] marks the coefficients that any cell reaches.
+// One wavefront per slot, lane = offset (all 64 busy at order 4), points in ascending order;
+// touch[c] marks the coefficients that any cell reaches.
 __global__ __launch_bounds__(256) void k_sf_cell_grad(SfAxes S, const int* __restrict__ nslot,
-                                                      const int* __restrict__ scell, const int* __restrict__ start,
-                                                      const int* __restrict__ list, const double* __restrict__ bN,
+                                                      const int* __restrict__ scell, const int2* __restrict__ slot,
+                                                      const int* __restrict__ start, const int* __restrict__ list,
+                                                      const double* __restrict__ bN,
                                                       const double* __restrict__ wss, const double* __restrict__ wdr,
                                                       double* __restrict__ part, uint8_t* __restrict__ touch) {
   const int s = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * 256 + threadIdx.x) >> 6));
   if (s >= *nslot) return;  // whole wavefronts
   const int k = S.a[0].k, ncx = S.a[0].nc, ncy = S.a[1].nc, ncz = S.a[2].nc, kk = k * k * k;
-  const int c = scell[s], b = start[c], e = start[c + 1];
+  const int c = scell[s], b = start[c] + (s - slot[c].x) * kSfChunk, e = min(start[c + 1], b + kSfChunk);
   const int cx = c % ncx, cy = (c / ncx) % ncy, cz = c / (ncx * ncy);
   for (int w = threadIdx.x & 63; w < kk; w += 64) {
     const int i = w % k, j = (w / k) % k, l = w / (k * k);
@@ -608,13 +629,13 @@ __global__ __launch_bounds__(256) void k_sf_cell_grad(SfAxes S, const int* __res
 }
 
 // gss/gdr[c] = factor * the sums of the cells c - [0, k)^3 for c: lane l takes the window
-// offsets l, l + 64, ... and lane 0 sums the 64 lanes in a fixed butterfly order, so the
-// result does not depend on scheduling.  One wavefront per kSfGradC coefficients; those no
+// offsets l, l + 64, ..., a cell's slots in turn, and lane 0 sums the 64 lanes in a fixed
+// butterfly order, so the result does not depend on scheduling.  One wavefront per kSfGradC coefficients; those no
 // cell reaches (most of a large lattice) are only written.  Forming the point sums here,
 // lane = cell, left the lanes at their cells' different point counts: 2.6 ms on 128 cells
 // over 128 x 64 x 64 voxels, the two kernels together 0.27 ms.
 constexpr int kSfGradC = 8;
-__global__ __launch_bounds__(256) void k_sf_grad(SfAxes S, int64_t ncoef, const int* __restrict__ slot,
+__global__ __launch_bounds__(256) void k_sf_grad(SfAxes S, int64_t ncoef, const int2* __restrict__ slot,
                                                  const double* __restrict__ part, const uint8_t* __restrict__ touch,
                                                  double fss, double fdr, float* __restrict__ gss,
                                                  float* __restrict__ gdr) {
@@ -635,10 +656,11 @@ __global__ __launch_bounds__(256) void k_sf_grad(SfAxes S, int64_t ncoef, const 
     for (int w = lane; w < kk; w += 64) {
       const int bx = ci[0] - w % k, by = ci[1] - (w / k) % k, bz = ci[2] - w / (k * k);
       if (bx < 0 || by < 0 || bz < 0) continue;
-      const int s = slot[bx + (int64_t)ncx * (by + (int64_t)ncy * bz)];
-      if (s < 0) continue;
-      a_ss += part[2 * ((int64_t)s * kk + w)];
-      a_dr += part[2 * ((int64_t)s * kk + w) + 1];
+      const int2 s = slot[bx + (int64_t)ncx * (by + (int64_t)ncy * bz)];
+      for (int64_t q = s.x; q < s.y; ++q) {
+        a_ss += part[2 * (q * kk + w)];
+        a_dr += part[2 * (q * kk + w) + 1];
+      }
     }
     for (int o = 1; o < 64; o <<= 1) {
       a_ss += __shfl_xor(a_ss, o, 64);

@@ -5,6 +5,7 @@
 // scalars, copies out).
 #include <algorithm>
 #include <chrono>
+#include <climits>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -4218,7 +4219,6 @@ TOS_EXPORT int tos_surface_constraints(tos_ctx* c, const tos_surface_opts* o, to
       regrow(C, C.sf_cbsum, nsb);
       regrow(C, C.sf_cboff, nsb + 1);
       regrow(C, C.sf_slot, ncoef);
-      regrow(C, C.sf_scell, ncoef);
       regrow(C, C.sf_touch, ncoef);
       C.sf_ncoef = (int64_t)ncoef;
     }
@@ -4290,7 +4290,7 @@ TOS_EXPORT int tos_surface_constraints(tos_ctx* c, const tos_surface_opts* o, to
                        C.partial);
     hipLaunchKernelGGL(k_sf_fold, dim3(1), dim3(256), 0, C.stream, (const double*)C.partial, (int)nbp, 3, S_TMP0,
                        C.scal);
-    // points grouped by knot cell: count, scan, slots; their number comes with the values below
+    // points grouped by knot cell: count, scan, slots; the number of slots comes with the values below
     if (C.sf_bcap < std::max<int64_t>(n, 1)) {
       const int64_t bcap = std::max<int64_t>(n, 1024) * 2;
       C.sf_bcap = 0;
@@ -4302,6 +4302,13 @@ TOS_EXPORT int tos_surface_constraints(tos_ctx* c, const tos_surface_opts* o, to
       C.sf_bcap = bcap;
     }
     const int64_t nc64 = (int64_t)ncoef, kk = (int64_t)C.sp_order * C.sp_order * C.sp_order;
+    const int64_t max_slots = std::min<int64_t>(n, nc64) + n / kSfChunk;
+    if (C.sf_scap < max_slots) {
+      const int64_t scap = 2 * max_slots;
+      C.sf_scap = 0;
+      regrow(C, C.sf_scell, scap);
+      C.sf_scap = scap;
+    }
     int* const nslot = (int*)(C.scal + S_SLOTS);
     hipLaunchKernelGGL(k_zero<int>, dim3(nblk(nc64)), dim3(256), 0, C.stream, C.sf_ccnt, nc64);
     if (n) {
@@ -4347,7 +4354,7 @@ TOS_EXPORT int tos_surface_constraints(tos_ctx* c, const tos_surface_opts* o, to
       dr_val = o->drip_mode <= 1 ? -1.0 : dr_sum / cnt_dr;
       dr_fac = o->drip_mode >= 6 ? 1.0 / cnt_dr : 0.0;
     }
-    // the points of a cell in order, the sums of every occupied cell, and the gather over the cells
+    // the points of a cell in order, the sums of every slot, and the gather over the cells
     if (C.sf_pcap < 2 * kk * slots) {
       const int64_t pcap = 2 * kk * (slots + slots / 2);
       C.sf_pcap = 0;
@@ -4360,13 +4367,15 @@ TOS_EXPORT int tos_surface_constraints(tos_ctx* c, const tos_surface_opts* o, to
       hipLaunchKernelGGL(k_sf_cell_fill, dim3(nblk(n)), dim3(256), 0, C.stream, n, (const int*)C.sf_key,
                          (const int*)C.sf_cstart, C.sf_ccnt, C.sf_list);
       hipLaunchKernelGGL(k_sf_cell_sort, dim3(nblk(64 * (int64_t)slots)), dim3(256), 0, C.stream, (const int*)nslot,
-                         (const int*)C.sf_scell, (const int*)C.sf_cstart, (const int*)C.sf_list, C.sf_sorted);
+                         (const int*)C.sf_scell, (const int2*)C.sf_slot, (const int*)C.sf_cstart, (const int*)C.sf_list,
+                         C.sf_sorted);
       hipLaunchKernelGGL(k_sf_cell_grad, dim3(nblk(64 * (int64_t)slots)), dim3(256), 0, C.stream, S, (const int*)nslot,
-                         (const int*)C.sf_scell, (const int*)C.sf_cstart, (const int*)C.sf_sorted, (const double*)C.sf_bN, (const double*)C.sf_wss,
+                         (const int*)C.sf_scell, (const int2*)C.sf_slot, (const int*)C.sf_cstart,
+                         (const int*)C.sf_sorted, (const double*)C.sf_bN, (const double*)C.sf_wss,
                          (const double*)C.sf_wdr, C.sf_part, C.sf_touch);
     }
     hipLaunchKernelGGL(k_sf_grad, dim3(nblk((nc64 + kSfGradC - 1) / kSfGradC * 64)), dim3(256), 0, C.stream, S, nc64,
-                       (const int*)C.sf_slot, (const double*)C.sf_part, (const uint8_t*)C.sf_touch, ss_fac, dr_fac,
+                       (const int2*)C.sf_slot, (const double*)C.sf_part, (const uint8_t*)C.sf_touch, ss_fac, dr_fac,
                        C.sscsens, C.dripcsens);
     LAUNCH_CHECK();
     HIPCHK(hipStreamSynchronize(C.stream));

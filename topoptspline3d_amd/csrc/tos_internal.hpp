@@ -256,9 +256,11 @@ struct Ctx {
   int* sf_key = nullptr;     // per point: knot cell (grown with sf_bidx)
   int* sf_list = nullptr;    // points grouped by knot cell, in arrival and in point order
   int* sf_sorted = nullptr;
-  int *sf_slot = nullptr, *sf_scell = nullptr;  // occupied cells: slot of a cell (-1 empty), cell of a slot
+  int2* sf_slot = nullptr;                      // first and end slot of a knot cell
+  int* sf_scell = nullptr;                      // cell of a slot
+  int64_t sf_scap = 0;                          // slots sf_scell holds
   uint8_t* sf_touch = nullptr;                  // coefficients reached by any point
-  double* sf_part = nullptr;                    // k^3 pairs of gradient sums per occupied cell
+  double* sf_part = nullptr;                    // k^3 pairs of gradient sums per slot
   int64_t sf_pcap = 0;                          // doubles in sf_part
   int64_t sf_bcap = 0;
   int64_t sf_ncoef = 0;      // coefficient count the per-coefficient buffers below are sized for
@@ -320,7 +322,7 @@ enum {
   S_RIG0,                            // 6 slots: R^T v of a rigid-motion projection
   S_AH0 = S_RIG0 + 6,                // 4 slots: alpha of the directions in the four direction
                                      // buffers of the precision-3 FCG
-  S_SLOTS = S_AH0 + 4,               // an int: number of occupied knot cells (k_sf_cell_slots)
+  S_SLOTS = S_AH0 + 4,               // an int: slots of the occupied knot cells (k_sf_cell_slots)
   S_COUNT = 40
 };
 static_assert(S_SLOTS < S_COUNT, "scalar slots");
