@@ -207,29 +207,42 @@ SOLVERS = {0: "FP64 V-cycle", 1: "FP32 V-cycle", 2: "FP32 V-cycle on FP16 coarse
            3: "FP32 V-cycle on FP16 coarse stencils, FP32 residual and K p"}
 
 
-def roofline(stats, info, n_active_nodes, steps, workload_tag=None, precision=1, sweep_mode=0):
+def rows_of_one_segment(flags, dims):
+    """Whether every grid row of free nodes fits one wave of the two-colour sweeps, 126 nodes
+    from a first node of either parity (FP64 cycles pair two fine colours per launch only then).
+    flags: node flags of a level of dims elements, bit 2 = free."""
+    free = (flags.reshape(dims[2] + 1, dims[1] + 1, dims[0] + 1) & 4) != 0
+    rows = free[free.any(axis=2)]
+    first, last = rows.argmax(axis=1), rows.shape[1] - 1 - rows[:, ::-1].argmax(axis=1)
+    return bool((last - first + 2 <= 126).all())
+
+
+def roofline(stats, info, n_active_nodes, steps, workload_tag=None, precision=1, sweep_mode=0, pairs_f64=False):
     """Roofline of the dominant kernel class (by total time among the classes with a
     single-level definition).  Algorithmic bytes per launch (each array read or written
     once at storage precision, index/flag re-reads excluded):
-      fine GS (FP32): one sweep = 4 N_e + (9*4 + 4) N_v; one launch = 1/8 (a colour) or,
-        with the in-wave paired schedule (sweep mode 3), 1/4 (two colours)
+      fine GS (FP32/FP64): one sweep = 4 N_e + (9 s + 4) N_v; one launch = 1/8 (a colour) or,
+        with the in-wave paired schedule (sweep mode 3; in FP64 where `pairs_f64`, rows of one
+        segment), 1/4 (two colours)
       fine residual (FP32/FP64):  4 N_e + (9 s + 4) N_v
       fine operator (FP64):       4 N_e + (6*8 + 4) N_v
-      level-1 stencil GS colour pass (FP32 cycle): (243*4 + 9*4) N_c1 / 8, or with the
-        FP16 stencil copy (precision 2) (122*4 + 4 + 9*4) N_c1 / 8"""
+      level-1 stencil GS pass (FP32 cycle): (243*4 + 9*4) N_c1 / 8, or with the FP16 stencil
+        copy (precision 2) (122*4 + 4 + 9*4) N_c1 / 8; twice that in sweep mode 3"""
     Ne, Nv = info["n_active_elements"][0], n_active_nodes
     Nc1 = info["n_free_nodes"][1] if info["n_levels"] > 1 else 0
-    colours = 2 if sweep_mode == 3 else 1  # colours per fine FP32 GS launch
+    colours = 2 if sweep_mode == 3 else 1  # colours per fine or level-1 FP32 GS launch
+    colours64 = colours if pairs_f64 else 1
     per_launch = {
         "fine_gs_f32": (4 * Ne + (9 * 4 + 4) * Nv) / 8.0 * colours,
-        "fine_gs_f64": (4 * Ne + (9 * 8 + 4) * Nv) / 8.0,
+        "fine_gs_f64": (4 * Ne + (9 * 8 + 4) * Nv) / 8.0 * colours64,
         "fine_resid_f32": 4 * Ne + (9 * 4 + 4) * Nv,
         "fine_resid_f64": 4 * Ne + (9 * 8 + 4) * Nv,
         "fine_apply_f64": 4 * Ne + (6 * 8 + 4) * Nv,
-        "st_gs_f32_l1": ((122 * 4 + 4 if precision >= 2 else 243 * 4) + 9 * 4) * Nc1 / 8.0,
+        "st_gs_f32_l1": ((122 * 4 + 4 if precision >= 2 else 243 * 4) + 9 * 4) * Nc1 / 8.0 * colours,
     }
-    flops = {"fine_gs_f32": 1170 * Nv / 8.0 * colours, "fine_gs_f64": 1170 * Nv / 8.0, "fine_resid_f32": 1152 * Nv,
-             "fine_resid_f64": 1152 * Nv, "fine_apply_f64": 1152 * Nv, "st_gs_f32_l1": 504 * Nc1 / 8.0}
+    flops = {"fine_gs_f32": 1170 * Nv / 8.0 * colours, "fine_gs_f64": 1170 * Nv / 8.0 * colours64,
+             "fine_resid_f32": 1152 * Nv, "fine_resid_f64": 1152 * Nv, "fine_apply_f64": 1152 * Nv,
+             "st_gs_f32_l1": 504 * Nc1 / 8.0 * colours}
     dom = max((k for k in stats if k in per_launch), key=lambda k: stats[k][0])
     tot = {k: v[0] for k, v in stats.items() if v[1] > 0}
     out = {"bound": "hbm", "peak": HBM_PEAK, "unit": "GB/s", "traffic": None, "kernel": dom,
@@ -241,7 +254,8 @@ def roofline(stats, info, n_active_nodes, steps, workload_tag=None, precision=1,
         js = json.load(open(tf))
         t = js.get("traffic")
         # (a GS profile holds for the schedule it was taken with)
-        if t and (not dom.startswith("fine_gs") or int(js.get("sweep_mode", 0)) == (sweep_mode if dom == "fine_gs_f32" else 0)):
+        mode = 0 if dom == "fine_gs_f64" and colours64 == 1 else sweep_mode
+        if t and (not dom.startswith("fine_gs") or int(js.get("sweep_mode", 0)) == mode):
             out["traffic"] = round(t["bytes_per_launch"])
             out["traffic_source"] = os.path.relpath(tf, ROOT)
             if js.get("valu"):
@@ -562,6 +576,7 @@ def main():
     loop, ms, its, res_max = run("plain", args.precision, False, args.steps, keep=True, recycle=args.recycle)
     info = loop.ctx.info()
     nv = active_nodes(wl["solid"])
+    pairs_f64 = rows_of_one_segment(loop.ctx.node_flags(0), info["level_dims"][0])
     log(f"[bench] levels {info['n_levels']} dims {info['level_dims']} coarse dofs {info['coarse_dofs']}")
     # per-kernel HIP-event timing in separate, untimed iterations (two events per launch
     # would otherwise add host work to the timed region)
@@ -588,7 +603,7 @@ def main():
                    "pcg_iterations": its, "max_rel_res": res_max},
         "roofline": roofline(stats, info, nv, args.profile_steps,
                              "ellipsoids_511x320x320" if wl["name"] == "c2" else None, args.precision,
-                             args.sweep_mode),
+                             args.sweep_mode, pairs_f64),
     }
     ms_plain, its_plain = ms, its
     if args.recycle > 0 and not args.no_recycle_compare:
