@@ -156,7 +156,8 @@ __global__ __launch_bounds__(256) void k_sensitivity(LevelView L, const uint8_t*
 // plane is formed; waves without an active element skip it.  Both kernels walk the table in its
 // order (dz outermost: plane d holds the taps tp.s[d] .. tp.s[d + 1]) with FP64 sums, so they
 // give the same result (an inactive or outside tap adds exactly zero to both sums).  k_filter
-// serves radii of 4.5 and more, whose ring would not fit in LDS.
+// serves radii below 0.5 (one tap, nothing to share) and of 4.5 and more: H = 4 with 16 rows takes
+// 124 KB of the CU's 160 KB of LDS, H = 5 would fit with 8 rows (117 KB) and is not built.
 // The FP64 products bound large boxes, the number of columns small ones: `zc` (filter_planes)
 // is taken so that the fullest CU has the fewest planes to form and to fill its rings with.
 // us before (32 planes per workgroup always, the per-element kernel above H = 3; one output at
@@ -547,9 +548,11 @@ __device__ __forceinline__ void oc_flat_chunk(int64_t n, int64_t chunk, bool vec
 // update being monotone in the threshold), or all at the lower (upper) clamp at the lower
 // (upper) end, keeps its sum and reads no element: with a target that the move limit does not
 // reach nearly every block after the first trial.  A trial over all blocks now takes 37 us, one
-// over decided blocks 3; a call with a target out of reach 4.4 -> 0.34 ms.  state[b]: elements at the upper clamp at the
-// bracket's ends and in the last trial (-1: not known, or some not decided by a clamp), and the
-// number of elements that are neither inactive nor shell.
+// over decided blocks 3.  ms of a call at 2^24 elements before and now: 4.5 -> 0.35 with a target
+// out of reach (31 trials), with one within reach 2.6 -> 0.9 (17 trials, move limit 0.03) and 2.07 ->
+// 0.86 (13 trials, 0.1).  state[b]: elements at the upper clamp at the bracket's ends and in the
+// last trial (-1: not known, or some not decided by a clamp), and the number of elements that are
+// neither inactive nor shell.
 __global__ __launch_bounds__(256) void k_oc_trial_flat(int64_t n, int64_t chunk, const uint8_t* __restrict__ act,
                                                        const uint8_t* __restrict__ shell, const float* __restrict__ rho,
                                                        const float* __restrict__ s, double move, double damp,

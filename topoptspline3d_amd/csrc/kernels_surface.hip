@@ -630,10 +630,10 @@ __global__ __launch_bounds__(256) void k_sf_cell_grad(SfAxes S, const int* __res
 
 // gss/gdr[c] = factor * the sums of the cells c - [0, k)^3 for c: lane l takes the window
 // offsets l, l + 64, ..., a cell's slots in turn, and lane 0 sums the 64 lanes in a fixed
-// butterfly order, so the result does not depend on scheduling.  One wavefront per kSfGradC coefficients; those no
-// cell reaches (most of a large lattice) are only written.  Forming the point sums here,
-// lane = cell, left the lanes at their cells' different point counts: 2.6 ms on 128 cells
-// over 128 x 64 x 64 voxels, the two kernels together 0.27 ms.
+// butterfly order, so the result does not depend on scheduling.  One wavefront per kSfGradC
+// coefficients; those no cell reaches (most of a large lattice) are only written.  Forming the
+// point sums here, lane = cell, left the lanes at their cells' different point counts: 2.6 ms on
+// 128 cells over 128 x 64 x 64 voxels, the two kernels together 0.12 ms.
 constexpr int kSfGradC = 8;
 __global__ __launch_bounds__(256) void k_sf_grad(SfAxes S, int64_t ncoef, const int2* __restrict__ slot,
                                                  const double* __restrict__ part, const uint8_t* __restrict__ touch,

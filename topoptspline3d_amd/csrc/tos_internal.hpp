@@ -102,7 +102,7 @@ struct Level {
   int n_segw[4][2] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
   float* ub32 = nullptr;
   bool pair_ok = false;          // stencil level: row segments built (k_st_gs_pairw)
-  bool pair_single = false;      // ... and every row is one segment (no deferred nodes)
+  bool pair_single = false;      // any level: every row is one segment (no deferred nodes)
   void* ubuf = nullptr;          // deferred nodes of the stencil-level paired GS (3 NP doubles)
   int4* segp = nullptr;          // even-x segments of all rows (paired prolongation into this level)
   int n_segp = 0;
@@ -292,7 +292,7 @@ struct Ctx {
                                 // on first demand (FP64 cycles, tos_get_stencil)
   bool st64_valid = false;      // FP64 stencils and cinv match the current operator
   int sweep_mode = 3;           // fine GS: 0 colour passes, 1 colour-slab wavefront, 2 row pairs,
-                                // 3 in-wave pairs (FP32 cycles)
+                                // 3 in-wave pairs
   bool graph_replay = true;     // replay the captured FCG iteration body
   struct SolveGraph {           // captured FCG iteration body per solve configuration
     int precision, pre, post, sweep, gal;
