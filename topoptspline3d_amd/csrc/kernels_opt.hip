@@ -151,21 +151,25 @@ __global__ __launch_bounds__(256) void k_sensitivity(LevelView L, const uint8_t*
 // elements and marches it along z over `zc` planes, keeping the 2H + 1 element planes of the
 // current output plane, each with an H-element halo in x and y, in an LDS ring as
 // (value, 1) for active elements and (0, 0) otherwise; every thread forms TY / (threads / 64)
-// outputs per plane from LDS, sharing each tap's table entry, which is uniform over the
-// workgroup and read through the scalar cache.  The next plane's loads are in flight while a
-// plane is formed; waves without an active element skip it.  Both kernels walk the table in its
+// outputs per plane from LDS, sharing each tap's table entry, which is read from LDS too: scalar
+// loads of it waited for every LDS read before them, which made radii of 2.5 to 3.5 slower on
+// large boxes than an entry read from LDS for each output.
+// The next plane's loads are in flight while a plane is formed; waves without an active element
+// skip it.  Both kernels walk the table in its
 // order (dz outermost: plane d holds the taps tp.s[d] .. tp.s[d + 1]) with FP64 sums, so they
 // give the same result (an inactive or outside tap adds exactly zero to both sums).  k_filter
 // serves radii below 0.5 (one tap, nothing to share) and of 4.5 and more: H = 4 with 16 rows takes
 // 124 KB of the CU's 160 KB of LDS, H = 5 would fit with 8 rows (117 KB) and is not built.
 // The FP64 products bound large boxes, the number of columns small ones: `zc` (filter_planes)
 // is taken so that the fullest CU has the fewest planes to form and to fill its rings with.
-// us before (32 planes per workgroup always, the per-element kernel above H = 3; one output at
-// a time, no loads ahead) and now: 71x43x37 H = 3 314 -> 23, 128x64x64 H = 2 132 -> 20,
-// 256x128x128 H = 4 744 -> 327.
+// us with 32 planes per workgroup always, an entry read per output and no loads ahead (the
+// per-element kernel above H = 3) and now: 71x43x37 H = 3 489 -> 16, 128x64x64 H = 2 126 -> 10,
+// 256x128x128 H = 4 726 -> 241, 511x320x100 H = 3 753 -> 580 (865 with entries by scalar loads),
+// 511x320x320 H = 3 2382 -> 1714 (2461).
 // ---------------------------------------------------------------------------------------
 constexpr int kFzX = 64;
 struct FilterPlanes { int s[10]; };
+struct alignas(16) FilterTap { double w; int o, unused; };
 
 template <int H, int TY>
 __global__ __launch_bounds__(TY <= 8 ? 256 : 512) void k_filter_zm(LevelView L, const uint8_t* __restrict__ eact,
@@ -177,6 +181,8 @@ __global__ __launch_bounds__(TY <= 8 ? 256 : 512) void k_filter_zm(LevelView L, 
   constexpr int NTH = TY <= 8 ? 256 : 512, ROWS = NTH / kFzX, R = TY / ROWS;
   constexpr int LX = kFzX + 2 * H, LY = TY + 2 * H, NZ = 2 * H + 1, PL = LX * LY, NL = (PL + NTH - 1) / NTH;
   __shared__ float2 ring[NZ * PL];
+  __shared__ FilterTap tab[NZ * NZ * NZ];
+  for (int i = threadIdx.x; i < tp.s[NZ]; i += NTH) tab[i] = FilterTap{wt[i], off[3 * i] + LX * off[3 * i + 1], 0};
   const int x0 = blockIdx.x * kFzX, y0 = blockIdx.y * TY, z0 = blockIdx.z * zc;
   const int nout = min(zc, L.ez - z0);
   const int tx = threadIdx.x % kFzX, ty = threadIdx.x / kFzX;  // rows ty + r ROWS
@@ -235,13 +241,12 @@ __global__ __launch_bounds__(TY <= 8 ? 256 : 512) void k_filter_zm(LevelView L, 
         const float2* pl = ring + sl * PL + c;
 #pragma unroll 4
         for (int i = tp.s[d]; i < tp.s[d + 1]; ++i) {
-          const int o = off[3 * i] + LX * off[3 * i + 1];
-          const double w = wt[i];
+          const FilterTap t = tab[i];
 #pragma unroll
           for (int r = 0; r < R; ++r) {
-            const float2 sv = pl[o + r * ROWS * LX];
-            gs[r] += w * (double)sv.x;
-            ws[r] += w * (double)sv.y;
+            const float2 sv = pl[t.o + r * ROWS * LX];
+            gs[r] += t.w * (double)sv.x;
+            ws[r] += t.w * (double)sv.y;
           }
         }
       }

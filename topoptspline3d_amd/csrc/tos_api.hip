@@ -3801,14 +3801,17 @@ TOS_EXPORT int tos_init_vol_sensitivity(tos_ctx* c) {
 }
 
 // Planes per workgroup of k_filter_zm over `cols` columns of ez planes: a workgroup forms zc
-// planes and fills its ring with 2H + 1 before the first (about a third of a plane's time
-// each); the fewest over the 256 CUs, the larger chunk among equals.
+// planes and fills its ring with 2H + 1 before the first (about a fifth of a plane's time each);
+// the fewest over the workgroups that fit the 256 CUs at once (8, 4, 2 and 1 a CU by LDS), the
+// larger chunk among equals.  Counting one a CU left the others idle: us of a call at r = 3.2,
+// 130x100x64 177 -> 121, 260x260x6 121 -> 81 (103 with 32 planes always).
 static int filter_planes(int cols, int ez, int H) {
+  const int fit = H == 1 ? 8 : (H == 2 ? 4 : (H == 3 ? 2 : 1));
   int best = 1;
   double cost = 0;
   for (int zc = 1; zc <= 32; ++zc) {
-    const int64_t blocks = (int64_t)cols * ((ez + zc - 1) / zc);
-    const double t = (double)((blocks + 255) / 256) * (zc + 0.35 * (2 * H + 1));
+    const int64_t blocks = (int64_t)cols * ((ez + zc - 1) / zc), slots = 256 * fit;
+    const double t = (double)((blocks + slots - 1) / slots) * (zc + 0.2 * (2 * H + 1));
     if (zc == 1 || t <= cost) { cost = t; best = zc; }
   }
   return best;
