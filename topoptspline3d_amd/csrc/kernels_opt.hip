@@ -155,11 +155,12 @@ __global__ __launch_bounds__(256) void k_sensitivity(LevelView L, const uint8_t*
 // loads of it waited for every LDS read before them, which made radii of 2.5 to 3.5 slower on
 // large boxes than an entry read from LDS for each output.
 // The next plane's loads are in flight while a plane is formed; waves without an active element
-// skip it.  Both kernels walk the table in its
-// order (dz outermost: plane d holds the taps tp.s[d] .. tp.s[d + 1]) with FP64 sums, so they
-// give the same result (an inactive or outside tap adds exactly zero to both sums).  k_filter
-// serves radii below 0.5 (one tap, nothing to share) and of 4.5 and more: H = 4 with 16 rows takes
-// 124 KB of the CU's 160 KB of LDS, H = 5 would fit with 8 rows (117 KB) and is not built.
+// skip it.  Both kernels walk the table in its order (dz outermost: plane d holds the taps
+// tp.s[d] .. tp.s[d + 1]) with FP64 sums, so they give the same result (an inactive or outside
+// tap adds exactly zero to both sums).  k_filter serves radii below 0.5 (one tap, nothing to
+// share), of 4.5 and more (H = 4 with 16 rows takes 136 KB of the CU's 160 KB of LDS; H = 5 would
+// fit with 8 rows, 138 KB, and is not built), and at H = 4 boxes that fill few lanes of a column
+// (filter_ring4).
 // The FP64 products bound large boxes, the number of columns small ones: `zc` (filter_planes)
 // is taken so that the fullest CU has the fewest planes to form and to fill its rings with.
 // us with 32 planes per workgroup always, an entry read per output and no loads ahead (the

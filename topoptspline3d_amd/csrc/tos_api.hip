@@ -3805,7 +3805,7 @@ TOS_EXPORT int tos_init_vol_sensitivity(tos_ctx* c) {
 // the fewest over the workgroups that fit the 256 CUs at once (8, 4, 2 and 1 a CU by LDS), the
 // larger chunk among equals.  Counting one a CU left the others idle: us of a call at r = 3.2,
 // 130x100x64 177 -> 121, 260x260x6 121 -> 81 (103 with 32 planes always).
-static int filter_planes(int cols, int ez, int H) {
+static int filter_planes(int cols, int ez, int H, double* planes = nullptr) {
   const int fit = H == 1 ? 8 : (H == 2 ? 4 : (H == 3 ? 2 : 1));
   int best = 1;
   double cost = 0;
@@ -3814,7 +3814,20 @@ static int filter_planes(int cols, int ez, int H) {
     const double t = (double)((blocks + slots - 1) / slots) * (zc + 0.2 * (2 * H + 1));
     if (zc == 1 || t <= cost) { cost = t; best = zc; }
   }
+  if (planes) *planes = cost;
   return best;
+}
+
+// Whether k_filter_zm<4> beats k_filter, which forms elements and not columns of 64 x 16 lanes: it
+// takes about as long as 3.2 planes of the ring kernel per plane's worth of elements on every CU,
+// and 3.5 for its own chain of taps (fitted to 442 boxes of 8 to 260 elements along x and y and 2 to
+// 1500 along z; the slower one is never taken where they differ by over 5 %).  us of a call at r =
+// 4.4, ring / per element: 8x100x1500 1110 / 494, 16x40x1500 518 / 403, 32x8x1500 213 / 214, 64x64x64
+// 76 / 171.  Below H = 4 the ring won on every one of these boxes.
+static bool filter_ring4(const LevelView& v) {
+  double planes = 0;
+  filter_planes(((v.ex + kFzX - 1) / kFzX) * ((v.ey + 15) / 16), v.ez, 4, &planes);
+  return planes <= 3.5 + 3.2 * ((double)v.ex * v.ey * v.ez / (256 * 1024));
 }
 
 TOS_EXPORT int tos_filter(tos_ctx* c, int which, double R) {
@@ -3866,7 +3879,7 @@ TOS_EXPORT int tos_filter(tos_ctx* c, int which, double R) {
     else if (Ri == 1) GO(1, 8)
     else if (Ri == 2) GO(2, 8)
     else if (Ri == 3) GO(3, 8)
-    else if (Ri == 4) GO(4, 16)
+    else if (Ri == 4 && filter_ring4(v)) GO(4, 16)
     else
       hipLaunchKernelGGL(k_filter, dim3(nblk(n)), dim3(256), 0, c->stream, v, ea, sb, b, (const int*)doff,
                          (const double*)dwt, nt);
