@@ -3820,8 +3820,8 @@ static int filter_planes(int cols, int ez, int H, double* planes = nullptr) {
 
 // Whether k_filter_zm<4> beats k_filter, which forms elements and not columns of 64 x 16 lanes: it
 // takes about as long as 3.2 planes of the ring kernel per plane's worth of elements on every CU,
-// and 3.5 for its own chain of taps (fitted to 442 boxes of 8 to 260 elements along x and y and 2 to
-// 1500 along z; the slower one is never taken where they differ by over 5 %).  us of a call at r =
+// and 3.5 for its own chain of taps (fitted to 221 boxes of 8 to 260 elements along x and y and 2 to
+// 1500 along z at two radii; the slower one is never taken where they differ by over 5 %).  us of a call at r =
 // 4.4, ring / per element: 8x100x1500 1110 / 494, 16x40x1500 518 / 403, 32x8x1500 213 / 214, 64x64x64
 // 76 / 171.  Below H = 4 the ring won on every one of these boxes.
 static bool filter_ring4(const LevelView& v) {
